@@ -23,12 +23,24 @@
 //   treat_error on the faces of row k-2
 //   the second continuity of row k-3              (continuity at t + dt)
 // and stores row k-3 of the new state.  Values of a row are carried in
-// registers while they are needed (7-row window); east/west neighbours are
-// DPP lane moves, made afresh in the row that uses them rather than carried
-// to the next one, and the face depths of row k-1 are derived where they are
-// used: register pressure sets the waves per SIMD.  No LDS staging and no
+// registers while they are needed; east/west neighbours are DPP lane moves,
+// made afresh in the row that uses them rather than carried to the next one:
+// register pressure sets the waves per SIMD.  No LDS staging and no
 // barriers: each wave is independent.  The grid is one wave per tile plus the
 // bookkeeping waves.
+//
+// What bounds it: issue of vector instructions (FP32 and mixed forms), the
+// latency of chains of FP64 operations at two waves per SIMD (FP64 form).  So
+// the row is written for few vector instructions: the conditions are lane
+// masks on the scalar unit, rows are addressed by a scalar offset, each
+// upwind product is formed once (the south one of a row is the north one of
+// the next, the east one of a cell the west one of its east neighbour), the
+// weirs, the momentum update and the first continuity run only in rows where
+// a lane needs them, and a row without fluxes and sources keeps its depths.
+// Measured per launch against per-lane booleans and every product formed
+// twice, results equal bit for bit: 48 grids of 128^2..1024^2 in FP32 145 ->
+// 121 us, 24 of them in FP64 217 -> 197 us; one 2048^2 grid FP32 91 -> 79,
+// FP64 161 -> 146 us.
 //
 // T is the type of the fluxes and of the momentum arithmetic, TH that of the
 // depths, the continuity updates and every switch that tests a depth.
@@ -44,50 +56,118 @@
 
 namespace sw2d {
 
-// bit of lane-1 of a wave-wide predicate
-__device__ __forceinline__ bool west_bit(bool p, int lane)
-{
-    unsigned long long m = __ballot(p);
-    return lane > 0 && ((m >> (lane - 1)) & 1ULL);
-}
+// Wave-wide predicates are kept as 64-bit lane masks in scalar registers: a
+// comparison writes one directly, the logic between them (which face is
+// active, which of the flux's branches applies, the west neighbour's bit) runs
+// on the scalar unit, and lanes() turns a mask back into the per-lane
+// condition of a select at no cost.  Per-lane booleans carried from row to row
+// or across a branch cost two vector instructions at every vote (0/1 and back).
+typedef unsigned long long u64;
+__device__ __forceinline__ u64 vote(bool p) { return __builtin_amdgcn_ballot_w64(p); }
+__device__ __forceinline__ bool lanes(u64 m) { return __builtin_amdgcn_inverse_ballot_w64(m); }
 
-// One scenario array, read and written at 32-bit element offsets.  Buf =
-// true: through a buffer resource (base and range in scalar registers, a
-// 32-bit byte offset per lane: no per-lane 64-bit address arithmetic; cell
-// offsets stay below 2^29, which the host enforces, so byte offsets of
-// doubles fit).  Buf = false: a global-address-space pointer (SGPR base +
-// 64-bit VGPR offset).  Measured: buffers make the FP32 form's launches
-// 1-2% faster and the FP64 and mixed forms' 1-2% slower, so only the FP32
-// form uses them.
+// One scenario array, read and written through a buffer resource (base and
+// range in scalar registers): a lane's byte offset within the row stays in one
+// register for the whole tile and the row's byte offset is scalar, so a row
+// costs no address arithmetic on the vector unit.  Offsets stay below 2^32
+// (cells below 2^29, which the host enforces).  A lane outside the grid or the
+// tile's output columns has the offset kOutside, past the range of any array:
+// its loads return 0, which is the ghost value, and its stores are dropped.
 typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
-template <typename V, bool Buf> struct Arr;
-template <typename V> struct Arr<V, false> {
-    gptr<V> p;
-    __device__ explicit Arr(const void *q) : p((gptr<V>)const_cast<void *>(q)) {}
-    __device__ __forceinline__ V load(unsigned off) const { return p[off]; }
-    __device__ __forceinline__ void store(unsigned off, V v) const { p[off] = v; }
-};
-template <typename V> struct Arr<V, true> {
-    __amdgpu_buffer_rsrc_t r;
-    // range: the whole 32-bit offset space; 0x00020000: the 32-bit data
-    // format (a buffer with the invalid format reads zeros)
-    __device__ explicit Arr(const void *q)
-        : r(__builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(q), (short)0, -1, 0x00020000)) {}
-    __device__ __forceinline__ V load(unsigned off) const
+constexpr unsigned kOutside = 0xffffff80u;
+template <typename V> struct Arr {
+    void *p;
+    unsigned bytes;
+    __device__ Arr(const void *q, unsigned cells)
+        : p(const_cast<void *>(q)), bytes(cells * (unsigned)sizeof(V)) {}
+    // the resource for one row; on == false: an empty range, so that the row
+    // reads ghosts (its stores are dropped) without a branch around the access:
+    // a branch would make the count of accesses in flight unknown, and the
+    // next row's wait would cover the prefetched row as well.  0x00020000: the
+    // 32-bit data format (a buffer with the invalid format reads zeros)
+    __device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc(bool on) const
     {
-        if constexpr (sizeof(V) == 4)
-            return __builtin_bit_cast(V, __builtin_amdgcn_raw_buffer_load_b32(r, (int)(off * 4u), 0, 0));
-        else
-            return __builtin_bit_cast(V, __builtin_amdgcn_raw_buffer_load_b64(r, (int)(off * 8u), 0, 0));
+        return __builtin_amdgcn_make_buffer_rsrc(p, (short)0, on ? bytes : 0u, 0x00020000);
     }
-    __device__ __forceinline__ void store(unsigned off, V v) const
+    __device__ __forceinline__ V load(unsigned off, unsigned row, bool on) const
     {
-        if constexpr (sizeof(V) == 4)
-            __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, v), r, (int)(off * 4u), 0, 0);
+        const unsigned ro = row * (unsigned)sizeof(V);
+        if constexpr (sizeof(V) == 1)
+            return __builtin_amdgcn_raw_buffer_load_b8(rsrc(on), (int)off, (int)ro, 0);
+        else if constexpr (sizeof(V) == 4)
+            return __builtin_bit_cast(V, __builtin_amdgcn_raw_buffer_load_b32(rsrc(on), (int)off, (int)ro, 0));
         else
-            __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, v), r, (int)(off * 8u), 0, 0);
+            return __builtin_bit_cast(V, __builtin_amdgcn_raw_buffer_load_b64(rsrc(on), (int)off, (int)ro, 0));
+    }
+    __device__ __forceinline__ void store(unsigned off, unsigned row, V v, bool on) const
+    {
+        const unsigned ro = row * (unsigned)sizeof(V);
+        if constexpr (sizeof(V) == 4)
+            __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, v), rsrc(on), (int)off, (int)ro, 0);
+        else
+            __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, v), rsrc(on), (int)off, (int)ro, 0);
     }
 };
+
+// New flux of a face between a cell ("o") and its north or west neighbour
+// ("b"), SW2D-EFDC.cu:97-353: the dry-bed weirs B1 (surface below the
+// neighbour's bed), B2 (the neighbour's below this bed) and B3 (one side dry)
+// all read (coef * hv) * sqrt(c2 * hv), every other face the momentum update
+// B4.  act: the faces to update (0 elsewhere); Wo, Wb: the sides' depths above
+// th; Lo, Lb: below it, so B3's "(h_o - th)(h_b - th) < 0" is mask logic.
+// mom(face depth, its B4 faces, surface difference, friction faces) gives B4.
+// FP32 depths test the water surfaces through the bed step dz = z_b - z_o,
+// FP64 ones through the elevations.
+template <typename T, typename TH, typename Mom>
+__device__ __forceinline__ T face_flux(const u64 act, const TH ho, const TH hb, const T dz,
+                                       const double zo, const double zb, const u64 Wo,
+                                       const u64 Wb, const u64 Lo, const u64 Lb, const TH thh,
+                                       const T gg, const Mom &mom)
+{
+    using M = num<T>;
+    constexpr bool kH32 = sizeof(TH) == 4;
+    u64 B1, B2;
+    double eo = 0, eb = 0;
+    if constexpr (kH32) {
+        B1 = vote(ho < dz);
+        B2 = vote(hb < -dz) & ~B1;
+    } else {
+        eo = ho + zo;
+        eb = hb + zb;
+        B1 = vote(eo < zb);
+        B2 = vote(eb < zo) & ~B1;
+    }
+    const u64 B3 = ((Wo & Lb) | (Lo & Wb)) & ~(B1 | B2);
+    const u64 weir = act & (B1 | B2 | B3), B4 = act & ~weir;
+    T val = 0;
+    if (weir) {
+        T coef = T(0.5440), hv = lanes(B2) ? (T)ho : (T)hb, c2 = gg;
+        if (B3 & act) {
+            T hv3;  // max(surfaces) - max(beds)
+            if constexpr (kH32)
+                hv3 = (dz <= T(0)) ? M::max_(ho, hb + dz) : M::max_(ho - dz, hb);
+            else
+                hv3 = (T)(__builtin_fmax(eo, eb) - __builtin_fmax(zo, zb));
+            coef = lanes(B3) ? T(0.350) : coef;
+            hv = lanes(B3) ? hv3 : hv;
+            c2 = lanes(B3) ? T(2.00) * gg : c2;
+        }
+        const T w = coef * hv * M::sqrt_(c2 * hv);
+        const u64 back = B2 | (B3 & Wo);  // flow toward the neighbour
+        const u64 wet = (B1 & Wb) | (B2 & Wo) | B3;
+        val = lanes(back) ? -w : w;
+        val = lanes(weir & wet) ? val : T(0);
+    }
+    if (B4) {
+        const TH hfd = TH(0.50) * (ho + hb);
+        T dsurf;
+        if constexpr (kH32) dsurf = (ho - hb) - dz;
+        else dsurf = (T)(eo - hb - zb);
+        const T up = mom((T)hfd, dsurf, B4 & vote(!(hfd <= thh)));
+        val = lanes(B4) ? up : val;
+    }
+    return val;
+}
 
 constexpr int kMaxTileRows = 512;
 
@@ -145,13 +225,6 @@ fused_step(const Scenario *__restrict__ scen, const TileRef *__restrict__ tiles,
         }
     }
     const int ib = k6 & 1;
-    // the state arrays (buffer resources in the FP32 form, see Arr); the
-    // Manning class bytes, read only with a map, through a global pointer
-    constexpr bool kBuf = sizeof(T) == 4 && sizeof(TH) == 4;
-    const Arr<TH, kBuf> h_out(d.st[ib ^ 1][0]);
-    const Arr<T, kBuf> um_out(d.st[ib ^ 1][1]), vn_out(d.st[ib ^ 1][2]);
-    const gptr<const uint8_t> clsg = (gptr<const uint8_t>)d.cls;
-
     if (tile >= d.ntiles) {
         PitchedState<T, TH> ps{(const TH *)d.st[ib][0], (const T *)d.st[ib][1],
                                (const T *)d.st[ib][2], s.R, s.C, d.P, (TH)s.th};
@@ -180,20 +253,58 @@ fused_step(const Scenario *__restrict__ scen, const TileRef *__restrict__ tiles,
     const int j = j0 - 3 + lane;
     const bool colin = (j >= 0) && (j < C);
     const bool colout = (lane >= 3) && (lane < 3 + d.W) && (j < C);
+    const u64 in_cols = vote(colin), out_cols = vote(colout);
     const int r0 = chunk * d.H;
     const int r1 = (r0 + d.H < R) ? r0 + d.H : R;
 
-    // CFL candidates only for an adaptive time step; a wave-uniform flag, so
-    // a scenario runs the same instructions alone and in a mixed batch
-    const bool adapt = kAdaptive && !s.fixed_dt;
-    const bool storm_on = kStorm && s.storm_on;
-    const bool map_on = kMap && s.ncls_on;
+    // software pipeline: row k+1 is loaded while row k is processed; the first
+    // row's loads are issued before the forcing is evaluated.  Rows and columns
+    // outside the grid read the ghost values 0 and are inactive.
+    const unsigned cells = (unsigned)R * (unsigned)P;
+    const Arr<TH> h_in(d.st[ib][0], cells), h_out(d.st[ib ^ 1][0], cells);
+    const Arr<T> um_in(d.st[ib][1], cells), um_out(d.st[ib ^ 1][1], cells);
+    const Arr<T> vn_in(d.st[ib][2], cells), vn_out(d.st[ib ^ 1][2], cells);
     // FP32 arithmetic: storm factors and source terms in FP32.  FP32 depths:
     // water-surface tests from bed differences carried per face (z stays
     // FP64 only to form them) and stochastically rounded depth updates.
     constexpr bool kF32 = sizeof(T) == 4;
     constexpr bool kH32 = sizeof(TH) == 4;
-    const T th = (T)s.th, gg = (T)s.g, dx = (T)s.dx, dy = (T)s.dy;
+    // the bed: FP64 elevations, or in the FP32 form the cell's bed-step pair
+    // (8 bytes as well; read as one double's bits); NaN marks an inactive cell
+    const Arr<const double> zg(kH32 ? d.dz : d.z, cells);
+    const bool map_on = kMap && s.ncls_on;
+    const Arr<uint8_t> cls_in(map_on ? (const void *)d.cls : (const void *)d.z, map_on ? cells : 0u);
+    __shared__ T nt_s[kMaxClasses];  // Manning coefficients of the classes
+    if (kMap && lane < kMaxClasses) nt_s[lane] = (T)s.ntab[lane];
+    const unsigned in1 = colin ? (unsigned)j : kOutside;
+    const unsigned inT = colin ? (unsigned)j * (unsigned)sizeof(T) : kOutside;
+    const unsigned inH = colin ? (unsigned)j * (unsigned)sizeof(TH) : kOutside;
+    const unsigned in8 = colin ? (unsigned)j * 8u : kOutside;
+    const unsigned outT = colout ? (unsigned)j * (unsigned)sizeof(T) : kOutside;
+    const unsigned outH = colout ? (unsigned)j * (unsigned)sizeof(TH) : kOutside;
+    const int kbeg = r0 - 3, kend = r1 + 3;
+    TH nh;
+    T nu, nv;
+    double nz;
+    uint8_t ncl;
+    auto load_row = [&](int k) {
+        const bool on = k >= 0 && k < R;
+        const unsigned row = on ? (unsigned)k * (unsigned)P : 0u;
+        nh = h_in.load(inH, row, on);
+        nu = um_in.load(inT, row, on);
+        nv = vn_in.load(inT, row, on);
+        nz = zg.load(in8, row, on);
+        if constexpr (kMap) ncl = cls_in.load(in1, row, on);
+        else ncl = 0;
+    };
+    load_row(kbeg);
+
+    // CFL candidates only for an adaptive time step; a wave-uniform flag, so
+    // a scenario runs the same instructions alone and in a mixed batch
+    const bool adapt = kAdaptive && !s.fixed_dt;
+    const bool storm_on = kStorm && s.storm_on;
+    const int nst = kSources ? s.nst : 0;
+    const T gg = (T)s.g, dx = (T)s.dx, dy = (T)s.dy;
     const TH thh = (TH)s.th;
     const T rdx = (T)(1.0 / s.dx), rdy = (T)(1.0 / s.dy);
     const T dt2 = (T)st.dt2;
@@ -228,290 +339,181 @@ fused_step(const Scenario *__restrict__ scen, const TileRef *__restrict__ tiles,
     const T rr1t = (T)rr1, rr2t = (T)rr2, ev1t = (T)ev1, ev2t = (T)ev2;
     const T P_lake = (T)s.P_lake, P_land = (T)s.P_land;
     const TH ewl = (TH)s.EV_WL_min;
+    // no water is added or taken in the second continuity: a row without
+    // fluxes then keeps its depths
+    const bool calm2 = !storm_on && nst == 0 && rr2 == 0.0 && ev2 == 0.0;
 
-    // outlet
-    const bool is_out_col = s.out_edge && (j == s.out_c);
+    // the outlet's row, where its column is among this wave's lanes, and its lane
+    const int ol = s.out_edge ? s.out_c - (j0 - 3) : -1;
+    const int orow = (ol >= 0 && ol < 64) ? s.out_r : -1000;
+    const u64 out_lane = 1ull << (ol & 63);
     T qo_eff = 0;
 
-    // carried rows: suffix 1 = row k-1, 2 = k-2, 3 = k-3
+    // carried rows: suffix 1 = row k-1, 2 = k-2, 3 = k-3.  Masks: A active,
+    // W deeper than th, L shallower
     TH h1 = 0, h2 = 0, h3 = 0;
-    double z1 = 0, z2 = 0, z1w = 0;
-    bool a1 = false, a2 = false, a3 = false, a1w = false;
-    T u1 = 0, u2 = 0, v1 = 0, v2 = 0;
-    T uu1_1 = 0, uu1_2 = 0;
-    T vv1_1 = 0, vv1_2 = 0;
-    T vva1 = 0;
+    double z1 = 0, z2 = 0;
+    u64 A1 = 0, A2 = 0, A3 = 0, W1 = 0, W2 = 0, L1 = 0, L2 = 0;
+    T u1 = 0, v1 = 0;
+    T uu1_1 = 0, vv1_1 = 0, vv1_2 = 0;
+    T px1 = 0, py1 = 0;    // upwind products between rows k-2 and k-1
     T dzn1 = 0, dzw1 = 0;  // FP32 form: z(k-2) - z(k-1) and z(k-1, j-1) - z(k-1, j)
     T nc1 = rn, nc2 = rn;
     T umnP = 0, vnnP = 0, umpP = 0, vnpP = 0;
-    bool dryP = false;
+    // faces that may carry flux: rows k-1, k-2, k-3 (north), k-2, k-3 (west)
+    u64 FXP = 0, FXQ = 0, FYP = 0, FYQ = 0;
+    u64 D1 = 0;  // cells of row k-3 that dried in the first continuity
 
-    double acc_vol = 0, acc_src = 0, acc_clip = 0, acc_q = 0;
+    double acc_vol = 0, acc_src = 0, acc_clip = 0;
     // CFL: the largest |u| + sqrt(g h) per direction; min_f dx / s_f = dx / max_f s_f
     // because rounding dx / s is monotone in s
     T smax_x = 0, smax_y = 0;
 
-    // software pipeline: row k+1 is loaded while row k is processed.  Rows
-    // outside the grid load a clamped row and are then replaced by the ghost
-    // values (0, inactive), so the loads need no branch.
-    const int kbeg = r0 - 3, kend = r1 + 3;
-    const int jc = colin ? j : (j < 0 ? 0 : C - 1);
-    const Arr<const TH, kBuf> h_in(d.st[ib][0]);
-    const Arr<const T, kBuf> um_in(d.st[ib][1]), vn_in(d.st[ib][2]);
-    // the bed: FP64 elevations, or in the FP32 form the cell's bed-step pair
-    // (8 bytes as well; read as one double's bits).  Ghosts read NaN either way.
-    const Arr<const double, kBuf> zg(kH32 ? d.dz : d.z);
-    const double zghost = kH32 ? __longlong_as_double(0x7FC000007FC00000LL) : __builtin_nan("");
-    auto load_row = [&](int k, TH &hh, T &uu, T &vv, double &zz, uint8_t &cc) {
-        const bool in = colin && k >= 0 && k < R;
-        const int kc = k < 0 ? 0 : (k >= R ? R - 1 : k);
-        const unsigned off = (unsigned)(kc * P + jc);
-        const TH lh = h_in.load(off);
-        const T lu = um_in.load(off), lv = vn_in.load(off);
-        const double lz = zg.load(off);
-        hh = in ? lh : TH(0);
-        uu = in ? lu : T(0);
-        vv = in ? lv : T(0);
-        zz = in ? lz : zghost;
-        cc = (map_on && in) ? clsg[off] : (uint8_t)0;
-    };
-    TH nh;
-    T nu, nv;
-    double nz;
-    uint8_t ncl;
-    load_row(kbeg, nh, nu, nv, nz, ncl);
-
+    // everything loaded so far is here (vmcnt, lgkmcnt 0): the loop's own waits
+    // then count only its own accesses
+    __builtin_amdgcn_s_waitcnt(0x0070);
     for (int k = kbeg; k < kend; ++k) {
         const TH h0 = nh;
         const T u0 = nu, v0 = nv;
         const double z0 = nz;
         const uint8_t cl0 = ncl;
-        load_row(k + 1, nh, nu, nv, nz, ncl);
+        load_row(k + 1);
         // FP32 form: z0 holds the bed steps of row k's cell to its north (low
         // word) and west (high word) neighbours, NaN for an inactive cell
         const u32x2 zsteps = __builtin_bit_cast(u32x2, z0);
-        const T zstep_n = (T)__uint_as_float(zsteps.x), zstep_w = (T)__uint_as_float(zsteps.y);
-        // inactive cells and ghosts carry NaN
-        const bool a0 = kH32 ? (zstep_w == zstep_w) : (z0 == z0);
-        // west/east neighbours of rows k-1 and k-2, made here rather than
-        // carried from the row before (shorter register live ranges)
-        const TH h1w = from_west(h1);
-        const T u1e = from_east(u1), u1w = from_west(u1);
-        const T v1e = from_east(v1), v1w = from_west(v1);
-        const T uu1_1w = from_west(uu1_1);
-        const T vv1_1e = from_east(vv1_1), vv1_2e = from_east(vv1_2), vv1_1w = from_west(vv1_1);
-        const T nc1w = map_on ? from_west(nc1) : rn;
-        const T nc0 = map_on ? (T)s.ntab[cl0] : rn;
+        const T dzn0 = (T)__uint_as_float(zsteps.x), dzw0 = (T)__uint_as_float(zsteps.y);
+        const u64 A0 = vote(kH32 ? (dzw0 == dzw0) : (z0 == z0)) & (k >= 0 && k < R ? in_cols : 0ull);
+        const u64 W0 = vote(h0 > thh), L0 = vote(h0 < thh);
+        T nc0 = rn;
+        if constexpr (kMap) nc0 = map_on ? nt_s[cl0] : rn;
 
         // ---- row k: face depths and velocities (hm_hn, uu1_vv1) ----
-        const TH h0w = from_west(h0);
-        const double z0w = from_west(z0);
-        const bool a0w = west_bit(a0, lane);
-        T dzn0 = 0, dzw0 = 0;
-        if constexpr (kH32) {
-            dzn0 = zstep_n;  // bed step across the north face of row k: (float)(z(k-1) - z(k))
-            dzw0 = zstep_w;  // bed step across the west face of row k: (float)(z(j-1) - z(j))
-        }
-        const TH hn0d = (j == 0) ? h0 : TH(0.50) * (h0 + h0w);
-        const TH hm0d = (k == 0) ? h0 : ((k == R) ? h1 : TH(0.50) * (h0 + h1));
+        // (row 0's north and column 0's west faces carry no flux, so their
+        // velocities are 0 whatever the face depth)
+        const TH hn0d = TH(0.50) * (h0 + from_west(h0));
+        const TH hm0d = TH(0.50) * (h0 + h1);
         const T hn0 = (T)hn0d, hm0 = (T)hm0d;
         const T uu1_0 = (hm0d >= thh) ? M::div_(u0, hm0) : T(0.00);
         const T vv1_0 = (hn0d >= thh) ? M::div_(v0, hn0) : T(0.0);
-        const T vv1_0e = from_east(vv1_0), vv1_0w = from_west(vv1_0);
-        const T uu1_0w = from_west(uu1_0);
-        // uua_vva (489-522): vva of row k, uua of row k-1
-        const T vva0 = (k > 0) ? T(0.250) * (vv1_0 + vv1_0e + vv1_1 + vv1_1e)
-                               : T(0.50) * (vv1_0 + vv1_0e);
-        const T uua1 = (j > 0) ? T(0.250) * (uu1_1 + uu1_0 + uu1_1w + uu1_0w)
-                               : T(0.50) * (uu1_1 + uu1_0);
 
-        if (adapt && colout && k >= r0 && k < r1) {
+        if (adapt && k >= r0 && k < r1) {
             // CFL candidates of the incoming state on the faces of row k
-            if (k >= 1 && a0 && a1 && hm0d > thh) {
+            if (lanes(A0 & A1 & out_cols & vote(hm0d > thh))) {
                 const T w = M::abs_(uu1_0) + M::sqrt_(gg * hm0);
                 smax_x = (w > smax_x) ? w : smax_x;
             }
-            if (j >= 1 && a0 && a0w && hn0d > thh) {
+            if (lanes(A0 & (A0 << 1) & out_cols & vote(hn0d > thh))) {
                 const T w = M::abs_(vv1_0) + M::sqrt_(gg * hn0);
                 smax_y = (w > smax_y) ? w : smax_y;
             }
+        }
+
+        // upwind products of the convection terms between rows f = k-1 and k:
+        // the south one of row f and the north one of row f + 1, so each is
+        // formed once and carried.  FP32: without the halvings (see dt2dx4)
+        const T uu1_0w = from_west(uu1_0);
+        T px0, py0;
+        if constexpr (kF32) {
+            const T sr = uu1_0 + uu1_1;
+            px0 = sr * (u0 + u1) + M::abs_(sr) * (u1 - u0);
+            const T sa = uu1_0 + uu1_0w;
+            py0 = sa * (v0 + v1) + M::abs_(sa) * (v1 - v0);
+        } else {
+            const T ur = T(0.50) * (uu1_0 + uu1_1);
+            px0 = ur * (u0 + u1) * T(0.50) + M::abs_(ur) * (u1 - u0) * T(0.50);
+            const T av = T(0.50) * (uu1_0 + uu1_0w);
+            py0 = av * (v0 + v1) * T(0.50) + M::abs_(av) * (v1 - v0) * T(0.50);
         }
 
         // ---- fluxes of row f = k-1 (flux, SW2D-EFDC.cu:97-353) ----
         const int f = k - 1;
         T umn = 0, vnn = 0;
         // rows before r0 - 1 feed no output row: the warm-up only builds the window
-        const bool flux_um = k >= r0, flux_vn = k >= r0 && k <= r1 + 1;
-        // x direction: um at the north face of (f, j); w = row f-1, e = row f.
-        // Dry-bed branches B1-B3 all read (coef * hv) * sqrt(c2 * hv); each of
-        // that and B4 (the momentum update) runs only when a lane needs it.
-        const bool act_x = flux_um && f > 0 && f < R && a1 && a2 && ((h2 > thh) || (h1 > thh));
-        if (__any(act_x)) {
-            // face depth of row k-1, derived as hm0 was for it
-            const TH hm1d = (k - 1 == 0) ? h1 : ((k - 1 == R) ? h2 : TH(0.50) * (h1 + h2));
-            const T hm1 = (T)hm1d;
-            const bool fr_x1 = !(hm1d <= thh);  // friction on: face depth above th
-            // water surfaces: FP64 (the reference's arithmetic) or, in the
-            // FP32 form, bed difference dz = z2 - z1 plus FP32 depths
-            bool b1, b2;
-            T dsurf, hv3;  // (h1 + z1) - (h2 + z2); max(surfaces) - max(beds)
-            if constexpr (kH32) {
-                const T dz = dzn1;
-                b1 = h1 < dz;
-                b2 = !b1 && (h2 < -dz);
-                dsurf = (h1 - h2) - dz;
-                hv3 = (dz <= T(0)) ? M::max_(h1, h2 + dz) : M::max_(h1 - dz, h2);
-            } else {
-                const double hhe = h1 + z1, hhw = h2 + z2;
-                b1 = hhe < z2;
-                b2 = !b1 && (hhw < z1);
-                dsurf = (T)(hhe - h2 - z2);
-                hv3 = (T)(__builtin_fmax(hhe, hhw) - __builtin_fmax(z1, z2));
-            }
-            const TH hhep = h1 - thh, hhwp = h2 - thh;
-            const bool b3 = !b1 && !b2 && (hhep * hhwp < 0);
-            const bool b4 = act_x && !b1 && !b2 && !b3;
-            T coef = T(0.5440), hv = (T)h2, c2 = gg;
-            bool wet = h2 > thh;
-            if (b2) { coef = T(-0.544); hv = (T)h1; wet = h1 > thh; }
-            if (b3) {
-                const T sgnm = (T)MH::sign_(hhep - hhwp);  // hhan / |hhan|
-                coef = -sgnm * T(0.350);
-                hv = hv3;
-                c2 = T(2.00) * gg;
-                wet = (h1 > 0) || (h2 > 0);
-            }
-            T val = 0;
-            if (__any(act_x && !b4)) val = wet ? coef * hv * M::sqrt_(c2 * hv) : T(0);
-            if (__any(b4)) {
+        // x direction: um at the north face of (f, j); w = row f-1, e = row f
+        // y direction: vn at the west face of (f, j); s = column j-1, n = column j
+        const u64 FX = k >= r0 ? A1 & A2 & (W1 | W2) : 0ull;
+        const u64 FY = (k >= r0 && k <= r1 + 1) ? A1 & (A1 << 1) & (W1 | (W1 << 1)) : 0ull;
+        if (FX) {
+            umn = face_flux<T, TH>(FX, h1, h2, dzn1, z1, z2, W1, W2, L1, L2, thh, gg,
+                                   [&](const T hm1, const T dsurf, const u64 fr) {
                 const T u13 = gg * hm1 * dt2dx * dsurf;
-                T u11, u12;
+                // the upwind product across the cell's west side; its east
+                // side's is the east neighbour's
+                const T u1w = from_west(u1);
+                T u11, u12, pd;
                 if constexpr (kF32) {
-                    // the halvings of the face velocities and of the upwind
-                    // products folded into dt2/(4 dx) and dt2/(4 dy)
-                    const T sr = uu1_0 + uu1_1, sl = uu1_1 + uu1_2;
-                    const T pr = sr * (u0 + u1) + M::abs_(sr) * (u1 - u0);
-                    const T pl = sl * (u1 + u2) + M::abs_(sl) * (u2 - u1);
-                    u11 = dt2dx4 * (pr - pl);
-                    const T su = vv1_1e + vv1_2e, sd = vv1_1 + vv1_2;
-                    const T pu = su * (u1e + u1) + M::abs_(su) * (u1 - u1e);
-                    const T pd = sd * (u1w + u1) + M::abs_(sd) * (u1w - u1);
-                    u12 = (j != 0) ? dt2dy4 * (pu - pd) : T(0);
+                    const T sd = vv1_1 + vv1_2;
+                    pd = sd * (u1w + u1) + M::abs_(sd) * (u1w - u1);
+                    u11 = dt2dx4 * (px0 - px1);
+                    u12 = dt2dy4 * (from_east(pd) - pd);
                 } else {
-                    const T ur = T(0.50) * (uu1_0 + uu1_1);
-                    const T ul = T(0.50) * (uu1_1 + uu1_2);
-                    const T umr = ur * (u0 + u1) * T(0.50) + M::abs_(ur) * (u1 - u0) * T(0.50);
-                    const T uml = ul * (u1 + u2) * T(0.50) + M::abs_(ul) * (u2 - u1) * T(0.50);
-                    u11 = dt2dx * (umr - uml);
-                    const T vu = T(0.50) * (vv1_1e + vv1_2e);
                     const T vd = T(0.50) * (vv1_1 + vv1_2);
-                    const T umu = vu * (u1e + u1) * T(0.50) + M::abs_(vu) * (u1 - u1e) * T(0.50);
-                    const T umd = vd * (u1w + u1) * T(0.50) + M::abs_(vd) * (u1w - u1) * T(0.50);
-                    u12 = (j != 0) ? dt2dy * (umu - umd) : T(0);
+                    pd = vd * (u1w + u1) * T(0.50) + M::abs_(vd) * (u1w - u1) * T(0.50);
+                    u11 = dt2dx * (px0 - px1);
+                    u12 = dt2dy * (from_east(pd) - pd);
                 }
+                u12 = (j != 0) ? u12 : T(0);
+                // uua_vva (489-522): vva of row f
+                const T vva1 = T(0.250) * (vv1_1 + from_east(vv1_1) + vv1_2 + from_east(vv1_2));
                 const T nf = map_on ? T(0.5) * (nc2 + nc1) : rn;
                 T ram = 0.00;
-                if (b4 && fr_x1) {
+                if (lanes(fr)) {
                     const T sqx = M::sqrt_(uu1_1 * uu1_1 + vva1 * vva1);
                     ram = M::div_(gg * nf * nf * sqx, pow1333(hm1));
                 }
-                T up;
                 if constexpr (kF32) {
                     const T a = dt2half * ram;
-                    up = M::div_((T(1.00) - a) * u1 + (-u11 - u12 - u13), T(1.00) + a);
+                    return M::div_((T(1.00) - a) * u1 + (-u11 - u12 - u13), T(1.00) + a);
                 } else {
-                    up = M::div_((T(1.00) - dt2 * ram * T(0.50)) * u1 + (-u11 - u12 - u13),
-                                 T(1.00) + dt2 * ram * T(0.50));
+                    return M::div_((T(1.00) - dt2 * ram * T(0.50)) * u1 + (-u11 - u12 - u13),
+                                   T(1.00) + dt2 * ram * T(0.50));
                 }
-                if (b4) val = up;
-            }
-            umn = act_x ? val : T(0);
+            });
         }
-        // y direction: vn at the west face of (f, j); s = column j-1, n = column j
-        const bool act_y = flux_vn && j > 0 && j < C && a1 && a1w && ((h1w > thh) || (h1 > thh));
-        if (__any(act_y)) {
-            const TH hn1d = (j == 0) ? h1 : TH(0.50) * (h1 + h1w);
-            const T hn1 = (T)hn1d;
-            const bool fr_y1 = !(hn1d <= thh);
-            bool b1, b2;
-            T dsurf, hv3;  // (h1 + z1) - (h1w + z1w); max(surfaces) - max(beds)
-            if constexpr (kH32) {
-                const T dz = dzw1;
-                b1 = h1 < dz;
-                b2 = !b1 && (h1w < -dz);
-                dsurf = (h1 - h1w) - dz;
-                hv3 = (dz <= T(0)) ? M::max_(h1, h1w + dz) : M::max_(h1 - dz, h1w);
-            } else {
-                const double hhn = h1 + z1, hhs = h1w + z1w;
-                b1 = hhn < z1w;
-                b2 = !b1 && (hhs < z1);
-                dsurf = (T)(hhn - h1w - z1w);
-                hv3 = (T)(__builtin_fmax(hhn, hhs) - __builtin_fmax(z1, z1w));
-            }
-            const TH hhnp = h1 - thh, hhsp = h1w - thh;
-            const bool b3 = !b1 && !b2 && (hhnp * hhsp < 0);
-            const bool b4 = act_y && !b1 && !b2 && !b3;
-            T coef = T(0.5440), hv = (T)h1w, c2 = gg;
-            bool wet = h1w > thh;
-            if (b2) { coef = T(-0.544); hv = (T)h1; wet = h1 > thh; }
-            if (b3) {
-                const T sgnm = (T)MH::sign_(hhnp - hhsp);
-                coef = -sgnm * T(0.350);
-                hv = hv3;
-                c2 = T(2.00) * gg;
-                wet = (h1 > 0) || (h1w > 0);
-            }
-            T val = 0;
-            if (__any(act_y && !b4)) val = wet ? coef * hv * M::sqrt_(c2 * hv) : T(0);
-            if (__any(b4)) {
+        if (FY) {
+            vnn = face_flux<T, TH>(FY, h1, from_west(h1), dzw1, z1, kH32 ? 0.0 : from_west(z1), W1,
+                                   W1 << 1, L1, L1 << 1, thh, gg,
+                                   [&](const T hn1, const T dsurf, const u64 fr) {
                 const T v13 = gg * hn1 * dt2dy * dsurf;
-                T v11, v12;
+                const T v1w = from_west(v1), uu1_1w = from_west(uu1_1);
+                T v11, v12, pd;
                 if constexpr (kF32) {
-                    const T sa = uu1_0 + uu1_0w, sb = uu1_1 + uu1_1w;
-                    const T pr = sa * (v0 + v1) + M::abs_(sa) * (v1 - v0);
-                    const T pl = sb * (v1 + v2) + M::abs_(sb) * (v2 - v1);
-                    v11 = (f != 0 && f != R) ? dt2dx4 * (pr - pl) : T(0);
-                    const T sp = vv1_1e + vv1_1, sq = vv1_1 + vv1_1w;
-                    const T pu = sp * (v1e + v1) + M::abs_(sp) * (v1 - v1e);
-                    const T pd = sq * (v1w + v1) + M::abs_(sq) * (v1w - v1);
-                    v12 = dt2dy4 * (pu - pd);
+                    const T sq = vv1_1 + from_west(vv1_1);
+                    pd = sq * (v1w + v1) + M::abs_(sq) * (v1w - v1);
+                    v11 = dt2dx4 * (py0 - py1);
+                    v12 = dt2dy4 * (from_east(pd) - pd);
                 } else {
-                    const T av = T(0.50) * (uu1_0 + uu1_0w);
-                    const T bv = T(0.50) * (uu1_1 + uu1_1w);
-                    const T vnr = av * (v0 + v1) * T(0.50) + M::abs_(av) * (v1 - v0) * T(0.50);
-                    const T vnl = bv * (v1 + v2) * T(0.50) + M::abs_(bv) * (v2 - v1) * T(0.50);
-                    v11 = (f != 0 && f != R) ? dt2dx * (vnr - vnl) : T(0);
-                    const T pv = T(0.50) * (vv1_1e + vv1_1);
-                    const T qv = T(0.50) * (vv1_1 + vv1_1w);
-                    const T vnu = pv * (v1e + v1) * T(0.50) + M::abs_(pv) * (v1 - v1e) * T(0.50);
-                    const T vnd = qv * (v1w + v1) * T(0.50) + M::abs_(qv) * (v1w - v1) * T(0.50);
-                    v12 = dt2dy * (vnu - vnd);
+                    const T qv = T(0.50) * (vv1_1 + from_west(vv1_1));
+                    pd = qv * (v1w + v1) * T(0.50) + M::abs_(qv) * (v1w - v1) * T(0.50);
+                    v11 = dt2dx * (py0 - py1);
+                    v12 = dt2dy * (from_east(pd) - pd);
                 }
-                const T nf = map_on ? T(0.5) * (nc1w + nc1) : rn;
+                v11 = (f != 0) ? v11 : T(0);
+                // uua_vva (489-522): uua of row f
+                const T uua1 = T(0.250) * (uu1_1 + uu1_0 + uu1_1w + uu1_0w);
+                const T nf = map_on ? T(0.5) * (from_west(nc1) + nc1) : rn;
                 T ram = 0.00;
-                if (b4 && fr_y1) {
+                if (lanes(fr)) {
                     const T sqy = M::sqrt_(uua1 * uua1 + vv1_1 * vv1_1);
                     ram = M::div_(gg * nf * nf * sqy, pow1333(hn1));
                 }
-                T up;
                 if constexpr (kF32) {
                     const T a = dt2half * ram;
-                    up = M::div_((T(1.00) - a) * v1 + (-v11 - v12 - v13), T(1.00) + a);
+                    return M::div_((T(1.00) - a) * v1 + (-v11 - v12 - v13), T(1.00) + a);
                 } else {
-                    up = M::div_((T(1.00) - dt2 * ram * T(0.50)) * v1 + (-v11 - v12 - v13),
-                                 T(1.00) + dt2 * ram * T(0.50));
+                    return M::div_((T(1.00) - dt2 * ram * T(0.50)) * v1 + (-v11 - v12 - v13),
+                                   T(1.00) + dt2 * ram * T(0.50));
                 }
-                if (b4) val = up;
-            }
-            vnn = act_y ? val : T(0);
+            });
         }
 
         // ---- first continuity of row g = k-2 at time t (602-664) ----
+        // it only decides which cells dry, so rows whose faces (their own and
+        // the next row's north ones) carry nothing skip it
         const int g = k - 2;
-        bool dryg = false;
-        T umpg = 0, vnpg = 0;
-        if (k >= r0 + 1) {
-            const T vnnPe = from_east(vnnP);
+        u64 D0 = 0;
+        T umpg = umnP, vnpg = vnnP;
+        if (k >= r0 + 1 && ((FX | FXP | FYP) || g == orow)) {
             const bool wet = h2 > ewl;
             const T Pc = wet ? P_lake : P_land;
             const T E = wet ? ev1t : T(0.000);
@@ -523,127 +525,134 @@ fused_step(const Scenario *__restrict__ scen, const TileRef *__restrict__ tiles,
                 else rr = storm1 ? (T)(s.st_peak * (gx1 * gy)) : T(0);
             }
             T ql = 0;
-            for (int i = 0; kSources && i < s.nst; ++i)
+            for (int i = 0; i < nst; ++i)
                 if (s.src_r[i] == g && s.src_c[i] == j) ql = (T)source_rate(s, i, st.t);
-            T ums = umn, umnn = umnP, vne = vnnPe, vnw = vnnP;
-            if (is_out_col && g == s.out_r) {
+            const T vnnPe = from_east(vnnP);
+            T du = umn - umnP, dv = vnnPe - vnnP;
+            if (g == orow) {
                 const T h2t = (T)h2;
-                const T qo = (h2 > thh) ? T(0.5440) * h2t * M::sqrt_(gg * h2t) : T(0);
-                if (s.out_edge == 1) ums = qo;
-                else if (s.out_edge == 2) umnn = -qo;
-                else if (s.out_edge == 3) vnw = -qo;
-                else vne = qo;
-                qo_eff = qo;
+                qo_eff = (h2 > thh) ? T(0.5440) * h2t * M::sqrt_(gg * h2t) : T(0);
+                const T du1 = qo_eff - umnP, du2 = umn - (-qo_eff);
+                const T dv3 = vnnPe - (-qo_eff), dv4 = qo_eff - vnnP;
+                if (s.out_edge <= 2) du = lanes(out_lane) ? (s.out_edge == 1 ? du1 : du2) : du;
+                else dv = lanes(out_lane) ? (s.out_edge == 3 ? dv3 : dv4) : dv;
             }
-            const T rhs = M::divc_(ums - umnn, dx, rdx) + M::divc_(vne - vnw, dy, rdy) - ql -
+            const T rhs = M::divc_(du, dx, rdx) + M::divc_(dv, dy, rdy) - ql -
                           rr * Pc + E;
             const TH hr = h2 - dt2h * (TH)rhs;
-            TH h1v = MH::max_(hr, TH(0.00));
-            if (!a2) h1v = 0.00;
-            dryg = a2 && (h1v < thh);
+            D0 = vote(MH::max_(hr, TH(0.00)) < thh) & A2;
             // ---- treat_error on the faces of row g (695-725) ----
-            umpg = umnP;
-            if (dryP && umpg > 0) umpg = 0;
-            if (dryg && umpg < 0) umpg = 0;
-            const bool drygw = west_bit(dryg, lane);
-            vnpg = vnnP;
-            if (drygw && vnpg > 0) vnpg = 0;
-            if (dryg && vnpg < 0) vnpg = 0;
-            if (is_out_col && g == s.out_r && dryg) qo_eff = 0;
+            if (D0 | D1) {
+                umpg = lanes((D1 & vote(umnP > 0)) | (D0 & vote(umnP < 0))) ? T(0) : umnP;
+                vnpg = lanes(((D0 << 1) & vote(vnnP > 0)) | (D0 & vote(vnnP < 0))) ? T(0) : vnnP;
+                if (g == orow) qo_eff = lanes(D0) ? T(0) : qo_eff;
+            }
         }
 
         // ---- second continuity of row q = k-3 at time t + dt; store ----
         const int q = k - 3;
-        if (k >= r0 + 3) {
-            const T vnpPe = from_east(vnpP);
-            const bool wet = h3 > ewl;
-            const T Pc = wet ? P_lake : P_land;
-            const T E = wet ? ev2t : T(0.000);
-            T rr = rr2t;
-            if (storm_on) {
-                const int qi = q - (r0 - 6);
-                const T gy = gy_s[1][qi < 0 ? 0 : qi];
-                if constexpr (kF32) rr = pk2 * gy;
-                else rr = storm2 ? (T)(s.st_peak * (gx2 * gy)) : T(0);
-            }
-            T ql = 0;
-            for (int i = 0; kSources && i < s.nst; ++i)
-                if (s.src_r[i] == q && s.src_c[i] == j) ql = (T)source_rate(s, i, st.tm);
-            T ums = umpg, umnn = umpP, vne = vnpPe, vnw = vnpP;
-            const bool outcell = is_out_col && q == s.out_r;
-            if (outcell) {
-                if (s.out_edge == 1) ums = qo_eff;
-                else if (s.out_edge == 2) umnn = -qo_eff;
-                else if (s.out_edge == 3) vnw = -qo_eff;
-                else vne = qo_eff;
-            }
-            const T rhs = M::divc_(ums - umnn, dx, rdx) + M::divc_(vne - vnw, dy, rdy) - ql -
-                          rr * Pc + E;
-            TH h2v;
-            double clip = 0.0;
-            if constexpr (kH32) {
-                // FP32 form: the depth update h3 - dt2 rhs is rounded
-                // stochastically.  TwoSum gives the exact rounding error er of
-                // sm = fl(h3 + tt); the result moves to the FP32 neighbour of sm
-                // on er's side with probability |er| / spacing, so rounding
-                // errors average out instead of adding up coherently (every
-                // cell of a uniformly wetted slope rounds the same small rain
-                // increment the same way).  The random number is a fixed hash
-                // of (cell, iteration): results are reproducible and do not
-                // depend on the tiling or on other scenarios.
-                const T tt = -dt2 * rhs;
-                const T sm = h3 + tt;
-                const T bp = sm - h3;
-                const T er = (h3 - (sm - bp)) + (tt - bp);
-                h2v = sm;
-                if (sm > T(0) && er != T(0)) {
-                    const uint32_t bits = __float_as_uint(sm);
-                    const T nb = __uint_as_float(er > T(0) ? bits + 1u : bits - 1u);
-                    const T pr = er * __builtin_amdgcn_rcpf(nb - sm);
-                    if (cell_uniform((uint32_t)(q * C + j), (uint32_t)it.step_index) < pr) h2v = nb;
-                }
-                // the exact update sm + er is negative iff sm < 0, or sm = 0 and
-                // er < 0 (|er| is at most half an ulp of sm); its FP64 value
-                // (exact: 48 bits suffice) is needed only then
-                if (sm < T(0) || (sm == T(0) && er < T(0))) {
-                    clip = -((double)sm + (double)er);
-                    h2v = 0;
-                }
+        const bool put = k >= r0 + 3;
+        TH h2v = 0;
+        if (put) {
+            if (calm2 && !(FXP | FXQ | FYQ) && q != orow && !vote(!(h3 >= TH(0)))) {
+                h2v = lanes(A3) ? h3 : TH(0);
+                if (lanes(A3 & out_cols)) acc_vol += (double)h2v;
             } else {
-                const TH hr = h3 - dt2h * (TH)rhs;
-                h2v = MH::max_(hr, TH(0.00));
-                if (hr < 0) clip = -(double)hr;
-            }
-            if (!a3) h2v = 0.00;
-            if (colout && q >= r0 && q < r1) {
-                const unsigned off = (unsigned)(q * P + j);
-                h_out.store(off, h2v);
-                um_out.store(off, umpP);
-                vn_out.store(off, vnpP);
-                if (a3) {
+                const bool wet = h3 > ewl;
+                const T Pc = wet ? P_lake : P_land;
+                const T E = wet ? ev2t : T(0.000);
+                T rr = rr2t;
+                if (storm_on) {
+                    const int qi = q - (r0 - 6);
+                    const T gy = gy_s[1][qi < 0 ? 0 : qi];
+                    if constexpr (kF32) rr = pk2 * gy;
+                    else rr = storm2 ? (T)(s.st_peak * (gx2 * gy)) : T(0);
+                }
+                T ql = 0;
+                for (int i = 0; i < nst; ++i)
+                    if (s.src_r[i] == q && s.src_c[i] == j) ql = (T)source_rate(s, i, st.tm);
+                const T vnpPe = from_east(vnpP);
+                T du = umpg - umpP, dv = vnpPe - vnpP;
+                if (q == orow) {
+                    const T du1 = qo_eff - umpP, du2 = umpg - (-qo_eff);
+                    const T dv3 = vnpPe - (-qo_eff), dv4 = qo_eff - vnpP;
+                    if (s.out_edge <= 2) du = lanes(out_lane) ? (s.out_edge == 1 ? du1 : du2) : du;
+                    else dv = lanes(out_lane) ? (s.out_edge == 3 ? dv3 : dv4) : dv;
+                }
+                const T rhs = M::divc_(du, dx, rdx) + M::divc_(dv, dy, rdy) - ql -
+                              rr * Pc + E;
+                const u64 sum = A3 & out_cols;
+                if constexpr (kH32) {
+                    // FP32 form: the depth update h3 - dt2 rhs is rounded
+                    // stochastically.  TwoSum gives the exact rounding error er of
+                    // sm = fl(h3 + tt); the result moves to the FP32 neighbour of sm
+                    // on er's side with probability |er| / spacing, so rounding
+                    // errors average out instead of adding up coherently (every
+                    // cell of a uniformly wetted slope rounds the same small rain
+                    // increment the same way).  The random number is a fixed hash
+                    // of (cell, iteration): results are reproducible and do not
+                    // depend on the tiling or on other scenarios.
+                    const T tt = -dt2 * rhs;
+                    const T sm = h3 + tt;
+                    const T bp = sm - h3;
+                    const T er = (h3 - (sm - bp)) + (tt - bp);
+                    h2v = sm;
+                    if (sm > T(0) && er != T(0)) {
+                        const uint32_t bits = __float_as_uint(sm);
+                        const T nb = __uint_as_float(er > T(0) ? bits + 1u : bits - 1u);
+                        const T pr = er * __builtin_amdgcn_rcpf(nb - sm);
+                        if (cell_uniform((uint32_t)(q * C + j), (uint32_t)it.step_index) < pr) h2v = nb;
+                    }
+                    // the exact update sm + er is negative iff sm < 0, or sm = 0 and
+                    // er < 0 (|er| is at most half an ulp of sm); its FP64 value
+                    // (exact: 48 bits suffice) is needed only then
+                    const u64 neg = vote(sm <= T(0)) & (vote(sm < T(0)) | vote(er < T(0)));
+                    if (neg) {
+                        if (lanes(neg & sum)) acc_clip += -((double)sm + (double)er);
+                        h2v = lanes(neg) ? TH(0) : h2v;
+                    }
+                } else {
+                    const TH hr = h3 - dt2h * (TH)rhs;
+                    h2v = MH::max_(hr, TH(0.00));
+                    const u64 neg = vote(hr < 0) & sum;
+                    if (neg) {
+                        if (lanes(neg)) acc_clip += -(double)hr;
+                    }
+                }
+                h2v = lanes(A3) ? h2v : TH(0.00);
+                if (lanes(sum)) {
                     acc_vol += (double)h2v;
                     if constexpr (kF32) acc_src += (double)(ql + rr * Pc - E);  // x dt2 below
                     else acc_src += st.dt2 * ((double)ql + (double)rr * (double)Pc - (double)E);
-                    acc_clip += clip;
                 }
-                if (outcell) acc_q += (double)qo_eff * s.dy;
             }
         }
+        const unsigned row = put ? (unsigned)q * (unsigned)P : 0u;
+        h_out.store(outH, row, h2v, put);
+        um_out.store(outT, row, umpP, put);
+        vn_out.store(outT, row, vnpP, put);
 
         // ---- rotate the row window ----
         h3 = h2; h2 = h1; h1 = h0;
-        z2 = z1; z1 = z0; z1w = z0w;
-        a3 = a2; a2 = a1; a1 = a0; a1w = a0w;
-        u2 = u1; u1 = u0;
-        v2 = v1; v1 = v0;
-        uu1_2 = uu1_1; uu1_1 = uu1_0;
+        z2 = z1; z1 = z0;
+        A3 = A2; A2 = A1; A1 = A0;
+        W2 = W1; W1 = W0;
+        L2 = L1; L1 = L0;
+        u1 = u0; v1 = v0;
+        uu1_1 = uu1_0;
         vv1_2 = vv1_1; vv1_1 = vv1_0;
-        vva1 = vva0;
+        px1 = px0; py1 = py0;
         dzn1 = dzn0; dzw1 = dzw0;
         nc2 = nc1; nc1 = nc0;
         umnP = umn; vnnP = vnn;
-        dryP = dryg; umpP = umpg; vnpP = vnpg;
+        umpP = umpg; vnpP = vnpg;
+        FXQ = FXP; FXP = FX;
+        FYQ = FYP; FYP = FY;
+        D1 = D0;
     }
+    // the outlet's discharge, where its cell is among this tile's outputs
+    double acc_q = 0;
+    if (orow >= r0 && orow < r1 && lanes(out_lane & out_cols)) acc_q = (double)qo_eff * s.dy;
 
     // ---- per-tile partial sums (fixed-order wave reductions) ----
     if constexpr (kF32) acc_src *= st.dt2;
