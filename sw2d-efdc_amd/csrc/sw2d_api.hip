@@ -468,7 +468,8 @@ int create_impl(const sw2d_grid_desc *grid, const double *z, const double *h0,
         return bail(rc);
     Clock ck[3];
     memset(ck, 0, sizeof(ck));
-    for (auto &c : ck) c.cfl_bits = kInfBits;
+    for (auto &c : ck)
+        for (auto &s : c.cfl) s.bits = kInfBits;
     ck[0].t = params->time0;
     e = hipMemcpy(h->clk, ck, sizeof(ck), hipMemcpyHostToDevice);
     if (e != hipSuccess) { hip_fail(h, e, "clock upload"); return bail(SW2D_E_HIP); }
@@ -938,7 +939,8 @@ int sw2d_time(sw2d_handle *h, double *time, long *mstep, double *dt2_next)
     if (mstep) *mstep = (long)h->host_mstep;
     if (dt2_next) {
         if (h->prm.adaptive) {
-            const double m = __builtin_bit_cast(double, ck.cfl_bits);
+            double m = INFINITY;
+            for (const auto &s : ck.cfl) m = std::min(m, __builtin_bit_cast(double, s.bits));
             const double d = h->prm.courant * m;
             const double mx = 2.00 * h->prm.dt;
             *dt2_next = (d < mx) ? d : mx;

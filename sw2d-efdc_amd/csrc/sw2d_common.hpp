@@ -11,18 +11,39 @@ struct StepTime {
     double t, dt, dt2, tm;
 };
 
-// start time and length of this iteration from the clock ring
+// the CFL minimum of a clock slot: one partial minimum a lane, combined over
+// the wave (all lanes active; the result is the same in every lane)
+__device__ __forceinline__ double clock_cfl(const Clock &ck)
+{
+    static_assert((kCflSlots & (kCflSlots - 1)) == 0 && kCflSlots <= 64, "");
+    double m = __longlong_as_double((long long)ck.cfl[threadIdx.x & (kCflSlots - 1)].bits);
+    for (int off = kCflSlots / 2; off >= 1; off >>= 1) {
+        const double o = __shfl_xor(m, off, 64);
+        m = (o < m) ? o : m;
+    }
+    const long long b = __double_as_longlong(m);  // uniform: into scalar registers
+    const unsigned lo = __builtin_amdgcn_readfirstlane((int)b), hi = __builtin_amdgcn_readfirstlane((int)(b >> 32));
+    return __longlong_as_double((long long)((unsigned long long)hi << 32 | lo));
+}
+// folds one wave's CFL minimum into it; i: any number that spreads the waves
+__device__ __forceinline__ void clock_note_cfl(Clock &ck, int i, double cfl)
+{
+    atomicMin(&ck.cfl[i & (kCflSlots - 1)].bits, (unsigned long long)__double_as_longlong(cfl));
+}
+
+// start time and length of this iteration from the clock ring; ADAPT false:
+// the step is known to be fixed
+template <bool ADAPT = true>
 __device__ __forceinline__ StepTime step_time(const StepCommon &s, const Iter &it)
 {
     const Clock &ck = s.clk[it.slot_a];
     StepTime st;
     st.t = ck.t;
-    if (s.fixed_dt) {
+    if (!ADAPT || s.fixed_dt) {
         st.dt = s.dt_fixed;
         st.dt2 = s.dt2_fixed;
     } else {
-        double m = __longlong_as_double((long long)ck.cfl_bits);
-        double d = s.courant * m;
+        double d = s.courant * clock_cfl(ck);
         st.dt2 = (d < s.dt2_max) ? d : s.dt2_max;
         st.dt = 0.5 * st.dt2;
     }
@@ -158,18 +179,22 @@ __device__ __forceinline__ void reduce_partials(const Partial *p, int n, int lan
                                                 double &src, double &clip, double &qo)
 {
     vol = 0; src = 0; clip = 0; qo = 0;
-    // four independent loads in flight per lane
-    int i = lane;
-    for (; i + 192 < n; i += 256) {
-        const Partial a = p[i], b = p[i + 64], c = p[i + 128], d = p[i + 192];
-        vol += a.vol; src += a.src; clip += a.clip; qo += a.qout;
-        vol += b.vol; src += b.src; clip += b.clip; qo += b.qout;
-        vol += c.vol; src += c.src; clip += c.clip; qo += c.qout;
-        vol += d.vol; src += d.src; clip += d.clip; qo += d.qout;
-    }
-    for (; i < n; i += 64) {
-        const Partial a = p[i];
-        vol += a.vol; src += a.src; clip += a.clip; qo += a.qout;
+    // One wave, so the latency of its loads is all there is: kInFlight records
+    // a lane are asked for before the first is added (past the end: record
+    // 0, added as zeros), in the order of one record after the other.
+    constexpr int kInFlight = 8;
+    for (int i = lane; i - lane < n; i += 64 * kInFlight) {
+        Partial a[kInFlight];
+#pragma unroll
+        for (int c = 0; c < kInFlight; c++) a[c] = p[i + 64 * c < n ? i + 64 * c : 0];
+#pragma unroll
+        for (int c = 0; c < kInFlight; c++) {
+            const bool in = i + 64 * c < n;
+            vol += in ? a[c].vol : 0.0;
+            src += in ? a[c].src : 0.0;
+            clip += in ? a[c].clip : 0.0;
+            qo += in ? a[c].qout : 0.0;
+        }
     }
     vol = wave_sum(vol); src = wave_sum(src); clip = wave_sum(clip); qo = wave_sum(qo);
 }
@@ -194,8 +219,8 @@ __device__ void bookkeeping(const StepCommon &s, const Iter &it, const StepTime 
         nb.t = st.tm + st.dt;
         nb.dt2_prev = st.dt2;
         nb.mstep = s.clk[it.slot_a].mstep + 2;
-        s.clk[it.slot_c].cfl_bits = kInfBits;
     }
+    if (lane < kCflSlots) s.clk[it.slot_c].cfl[lane].bits = kInfBits;
     if (it.step_index > 0) {
         double vol, src, clip, qo;
         reduce_partials(it.part_in, s.nparts, lane, vol, src, clip, qo);

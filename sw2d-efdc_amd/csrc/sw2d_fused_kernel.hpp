@@ -197,11 +197,11 @@ fused_step(const Scenario *__restrict__ scen, const TileRef *__restrict__ tiles,
         const int x = b % nx, i = b / nx;
         b = x * per + (x < rem ? x : rem) + i;
     }
-    int sid = 0, tile = b;
+    int sid = 0, local = b;
     if (tiles) {
         const TileRef t = tiles[b];
         sid = t.sid;
-        tile = t.local;
+        local = t.local;
     }
     // the descriptor is read in place (no local copy: its uniform fields stay
     // reloadable scalar loads instead of pinned registers)
@@ -215,16 +215,20 @@ fused_step(const Scenario *__restrict__ scen, const TileRef *__restrict__ tiles,
     it.part_out = d.part + (size_t)(k6 & 1) * s.nparts;
     it.part_in = d.part + (size_t)((k6 + 1) & 1) * s.nparts;
     it.step_index = s.clk[it.slot_a].mstep >> 1;
-    const StepTime st = step_time(s, it);
+    const StepTime st = step_time<kAdaptive>(s, it);
     if (d.status) {
         // batch member: a finished scenario leaves its blocks idle
         if (d.status->done) return;
         if (!(it.step_index < d.k_end && st.t + st.dt <= d.t_end)) {
-            if (tile == d.ntiles && lane == 0) d.status->done = 1;
+            if (local == 0 && lane == 0) d.status->done = 1;
             return;
         }
     }
     const int ib = k6 & 1;
+    // the bookkeeping waves come first, so that the reduction of the last
+    // iteration's partial sums runs beside the tiles and not after them
+    const int nbook = d.nblocks - d.ntiles;
+    const int tile = local < nbook ? d.ntiles + local : local - nbook;
     if (tile >= d.ntiles) {
         PitchedState<T, TH> ps{(const TH *)d.st[ib][0], (const T *)d.st[ib][1],
                                (const T *)d.st[ib][2], s.R, s.C, d.P, (TH)s.th};
@@ -233,7 +237,7 @@ fused_step(const Scenario *__restrict__ scen, const TileRef *__restrict__ tiles,
             ua = (double)ps.uua(r, j);
             va = (double)ps.vva(r, j);
         };
-        const int part = tile - d.ntiles;
+        const int part = local;
         bookkeeping(s, it, st, vel, part, lane);
         if (part == 0 && lane == 0 && d.status) {
             const long long kn = it.step_index + 1;
@@ -672,7 +676,7 @@ fused_step(const Scenario *__restrict__ scen, const TileRef *__restrict__ tiles,
         p.vol = acc_vol; p.src = acc_src; p.clip = acc_clip; p.qout = acc_q;
         it.part_out[tile] = p;
         if (adapt && cfl < INFINITY)
-            atomicMin(&s.clk[it.slot_b].cfl_bits, (unsigned long long)__double_as_longlong(cfl));
+            clock_note_cfl(s.clk[it.slot_b], tile, cfl);
     }
 }
 
@@ -711,7 +715,7 @@ __global__ void __launch_bounds__(256) init_cfl(const TH *h, const T *um, const 
     }
     cfl = wave_min(cfl);
     if ((threadIdx.x & 63) == 0 && cfl < INFINITY)
-        atomicMin(&clk[0].cfl_bits, (unsigned long long)__double_as_longlong(cfl));
+        clock_note_cfl(clk[0], blockIdx.x, cfl);
 }
 
 // one derived field of the current state (hm_hn, uu1_vv1, uu_vv, uua_vva) over

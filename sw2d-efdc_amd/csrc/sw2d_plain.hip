@@ -139,7 +139,7 @@ __global__ void __launch_bounds__(256) plain_flux(const PlainArgs a)
     if (ADAPT) {
         cfl = wave_min(cfl);
         if ((threadIdx.x & 63) == 0 && cfl < INFINITY)
-            atomicMin(&s.clk[s.slot_b].cfl_bits, (unsigned long long)__double_as_longlong(cfl));
+            clock_note_cfl(s.clk[s.slot_b], blockIdx.x, cfl);
     }
 }
 
@@ -345,7 +345,7 @@ __global__ void __launch_bounds__(256) plain_init(const PlainArgs a, int adaptiv
     if (adaptive) {
         cfl = wave_min(cfl);
         if ((threadIdx.x & 63) == 0 && cfl < INFINITY)
-            atomicMin(&a.s.clk[0].cfl_bits, (unsigned long long)__double_as_longlong(cfl));
+            clock_note_cfl(a.s.clk[0], blockIdx.x, cfl);
     }
 }
 
