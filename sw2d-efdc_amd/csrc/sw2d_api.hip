@@ -37,7 +37,7 @@ StepCommon make_common(sw2d_handle *h)
     s.rain = h->rain; s.nrain = h->nrain; s.dtrain = h->dtrain;
     s.evapo = h->evapo; s.nevapo = h->nevapo; s.evap_on = h->evap_on;
     s.Q = h->Q; s.nq = h->nq; s.nst = h->nst; s.dtoq = h->dtoq;
-    s.src_r = h->src_r; s.src_c = h->src_c;
+    s.src_r = h->src_r; s.src_c = h->src_c; s.src_rate = h->src_rate;
     s.storm_on = h->storm_on;
     s.st_peak = h->storm.peak; s.st_x0 = h->storm.x0; s.st_y0 = h->storm.y0;
     s.st_vx = h->storm.vx; s.st_vy = h->storm.vy; s.st_sigma = h->storm.sigma;
@@ -56,7 +56,7 @@ StepCommon make_common(sw2d_handle *h)
 
 bool fused(const sw2d_handle *h) { return h->prm.kernel == SW2D_KERNEL_FUSED; }
 
-int fused_blocks(const sw2d_handle *h) { return h->ntiles + 1 + (h->nbc + 63) / 64; }
+int fused_blocks(const sw2d_handle *h) { return h->ntiles + book_blocks(h->nbc); }
 
 // the fused kernel's descriptor of a stand-alone handle (phase 0 = iteration 0)
 Scenario make_scenario(sw2d_handle *h)
@@ -90,6 +90,7 @@ int upload_desc(sw2d_handle *h)
     if (!h->desc_dirty) return SW2D_OK;
     const Scenario d = make_scenario(h);
     HIPCHK(h, hipMemcpyAsync(h->dscen, &d, sizeof d, hipMemcpyHostToDevice, h->stream));
+    HIPCHK(h, launch_forcing(h->stream, h->dscen, 1));
     HIPCHK(h, hipStreamSynchronize(h->stream));
     h->desc_dirty = false;
     return SW2D_OK;
@@ -200,7 +201,7 @@ long wave_slots(int device, int prec, int features)
 int blocks_at(const sw2d_handle *h, int H)
 {
     const int nstrips = (h->C + h->W - 1) / h->W;
-    return nstrips * ((h->R + H - 1) / H) + 1 + (h->nbc + 63) / 64;
+    return nstrips * ((h->R + H - 1) / H) + book_blocks(h->nbc);
 }
 
 // Tile heights in [2, 128] that fill whole rounds of wave slots: for k = 1..6
@@ -250,10 +251,13 @@ void set_tiles(sw2d_handle *h, int H)
 
 int upload_source_cells(sw2d_handle *h, const int *rr, const int *cc, int n)
 {
-    dfree(h, h->src_r); dfree(h, h->src_c);
+    dfree(h, h->src_r); dfree(h, h->src_c); dfree(h, h->src_rate);
     h->src_r = h->src_c = nullptr;
+    h->src_rate = nullptr;
     int rc;
-    if ((rc = dalloc(h, &h->src_r, n)) || (rc = dalloc(h, &h->src_c, n))) return rc;
+    if ((rc = dalloc(h, &h->src_r, n)) || (rc = dalloc(h, &h->src_c, n)) ||
+        (rc = dalloc(h, &h->src_rate, 6 * (size_t)n)))
+        return rc;
     if (n > 0) {
         HIPCHK(h, hipMemcpy(h->src_r, rr, sizeof(int) * n, hipMemcpyHostToDevice));
         HIPCHK(h, hipMemcpy(h->src_c, cc, sizeof(int) * n, hipMemcpyHostToDevice));
@@ -712,6 +716,8 @@ static std::vector<int> fill_heights(const sw2d_handle *h)
 // height and retiles to the fastest (see sw2d_autotune)
 static int autotune_over(sw2d_handle *h, int iters, std::vector<int> cand, int *tile_rows)
 {
+    // the trials read the live clock, so its forcing has to be there
+    if (int rc = upload_desc(h)) return rc;
     HIPCHK(h, hipStreamSynchronize(h->stream));
     std::sort(cand.begin(), cand.end());
     cand.erase(std::unique(cand.begin(), cand.end()), cand.end());

@@ -117,8 +117,10 @@ int rebuild(sw2d_batch *b)
         BCHK(b, hipMalloc(&b->dtiles, sizeof(TileRef) * cap));
         b->tiles_cap = cap;
     }
-    if (top > 0)
+    if (top > 0) {
         BCHK(b, hipMemcpy(b->dscen, desc.data(), sizeof(Scenario) * top, hipMemcpyHostToDevice));
+        BCHK(b, launch_forcing(b->stream, b->dscen, top));
+    }
     if (!tiles.empty())
         BCHK(b, hipMemcpy(b->dtiles, tiles.data(), sizeof(TileRef) * tiles.size(), hipMemcpyHostToDevice));
     if ((int)tiles.size() != b->nblocks || features != b->features) bdrop_graph(b);
@@ -468,7 +470,7 @@ int sw2d_batch_autotune(sw2d_batch *b, int iters, int *tile_rows)
         // the smallest candidate
         const int hmin = h->prm.tile_rows > 0 ? h->prm.tile_rows : cand[0];
         sc[i].maxt = ((h->C + h->W - 1) / h->W) * ((h->R + hmin - 1) / hmin);
-        maxblocks += sc[i].maxt + 1 + (h->nbc + 63) / 64;
+        maxblocks += sc[i].maxt + book_blocks(h->nbc);
     }
     for (int i = 0; i < nm && !rc; i++) {
         sw2d_handle *h = b->members[i];

@@ -28,4 +28,17 @@ hipError_t launch_peek(sw2d_handle *h, const StepCommon &sc)
     return hipGetLastError();
 }
 
+// one wave a descriptor; a slot without a member is all zeros
+__global__ void __launch_bounds__(64) forcing_kernel(const Scenario *scen)
+{
+    const StepCommon &s = scen[blockIdx.x].s;
+    if (s.clk) note_forcing(s, s.slot_a, s.clk[s.slot_a].t, threadIdx.x);
+}
+
+hipError_t launch_forcing(hipStream_t stream, const Scenario *scen, int n)
+{
+    hipLaunchKernelGGL(forcing_kernel, dim3(n), dim3(64), 0, stream, scen);
+    return hipGetLastError();
+}
+
 }  // namespace sw2d

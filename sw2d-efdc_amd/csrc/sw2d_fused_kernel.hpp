@@ -238,7 +238,7 @@ fused_step(const Scenario *__restrict__ scen, const TileRef *__restrict__ tiles,
             va = (double)ps.vva(r, j);
         };
         const int part = local;
-        bookkeeping(s, it, st, vel, part, lane);
+        bookkeeping(s, it, st, vel, part, lane, true);
         if (part == 0 && lane == 0 && d.status) {
             const long long kn = it.step_index + 1;
             const double tn = st.tm + st.dt;
@@ -307,7 +307,18 @@ fused_step(const Scenario *__restrict__ scen, const TileRef *__restrict__ tiles,
     // a scenario runs the same instructions alone and in a mixed batch
     const bool adapt = kAdaptive && !s.fixed_dt;
     const bool storm_on = kStorm && s.storm_on;
-    const int nst = kSources ? s.nst : 0;
+    // the scenario's point sources, where one lies among the tile's columns and
+    // the rows of its first continuity
+    int nst = kSources ? s.nst : 0;
+    if (nst > 0) {
+        bool here = false;
+        for (int i = lane; i < nst; i += 64) {
+            const int r = s.src_r[i], c = s.src_c[i] - (j0 - 3);
+            here |= r >= r0 - 1 && r <= r1 && c >= 0 && c < 64;
+        }
+        if (!vote(here)) nst = 0;
+    }
+    const double *src_rate = s.src_rate + (size_t)it.slot_a * 2 * s.nst;
     const T gg = (T)s.g, dx = (T)s.dx, dy = (T)s.dy;
     const TH thh = (TH)s.th;
     const T rdx = (T)(1.0 / s.dx), rdy = (T)(1.0 / s.dy);
@@ -320,8 +331,11 @@ fused_step(const Scenario *__restrict__ scen, const TileRef *__restrict__ tiles,
     const T rn = (T)s.rn;
 
     // forcing of this iteration: first continuity at t, second at t + dt
-    const double rr1 = rain_rate(s, st.t), rr2 = rain_rate(s, st.tm);
-    const double ev1 = evap_rate(s, st.t), ev2 = evap_rate(s, st.tm);
+    // (note_forcing)
+    const Clock &ck = s.clk[it.slot_a];
+    const double rr1 = ck.force[0], ev1 = ck.force[2];
+    const double rr2 = adapt ? rain_rate(s, st.tm) : ck.force[1];
+    const double ev2 = adapt ? evap_rate(s, st.tm) : ck.force[3];
     const bool storm1 = storm_live(s, st.t), storm2 = storm_live(s, st.tm);
     double gx1 = 0, gx2 = 0;
     T pk1 = 0, pk2 = 0;  // FP32 form: peak * gx of this column, 0 outside the storm window
@@ -530,7 +544,7 @@ fused_step(const Scenario *__restrict__ scen, const TileRef *__restrict__ tiles,
             }
             T ql = 0;
             for (int i = 0; i < nst; ++i)
-                if (s.src_r[i] == g && s.src_c[i] == j) ql = (T)source_rate(s, i, st.t);
+                if (s.src_r[i] == g && s.src_c[i] == j) ql = (T)src_rate[2 * i];
             const T vnnPe = from_east(vnnP);
             T du = umn - umnP, dv = vnnPe - vnnP;
             if (g == orow) {
@@ -574,7 +588,8 @@ fused_step(const Scenario *__restrict__ scen, const TileRef *__restrict__ tiles,
                 }
                 T ql = 0;
                 for (int i = 0; i < nst; ++i)
-                    if (s.src_r[i] == q && s.src_c[i] == j) ql = (T)source_rate(s, i, st.tm);
+                    if (s.src_r[i] == q && s.src_c[i] == j)
+                        ql = (T)(adapt ? source_rate(s, i, st.tm) : src_rate[2 * i + 1]);
                 const T vnpPe = from_east(vnpP);
                 T du = umpg - umpP, dv = vnpPe - vnpP;
                 if (q == orow) {

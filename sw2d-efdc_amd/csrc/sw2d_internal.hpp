@@ -57,6 +57,8 @@ struct Clock {
     double t;                    // time at the start of the iteration reading this slot
     double dt2_prev;             // length of the iteration that wrote this slot
     long long mstep;             // reference half-step counter
+    double force[4];             // fused path: rain at t and at t + dt, evaporation at t and at
+                                 // t + dt (m/s; with an adaptive step the two at t only)
     CflSlot cfl[kCflSlots];      // CFL minimum (its partial minima)
 };
 
@@ -90,6 +92,7 @@ struct StepCommon {
     const double *evapo; int nevapo; int evap_on;
     const double *Q; int nq; int nst; double dtoq;
     const int *src_r; const int *src_c;
+    double *src_rate;            // fused path: [clock slot][source][at t, at t + dt] in m/s
     // extensions
     int storm_on;
     double st_peak, st_x0, st_y0, st_vx, st_vy, st_sigma, st_t0, st_t1;
@@ -147,13 +150,18 @@ struct Scenario {
     int W;                   // output columns per tile (64 - 6)
     int H;                   // output rows per tile
     int nstrips, ntiles;     // tiles of this scenario
-    int nblocks;             // tiles + bookkeeping waves
+    int nblocks;             // bookkeeping waves + tiles
     Partial *part;           // two halves of nparts records
     int phase0;              // launch phase of this scenario's iteration 0 (mod 6)
     long long k_end;         // a batch member stops before iteration k_end ...
     double t_end;            // ... or before an iteration that would end past t_end + dt
     Status *status;          // batch members only; NULL for a stand-alone handle
 };
+
+// bookkeeping waves besides those of the lake-inflow records (64 each): the
+// clock and the forcing, the ledger
+constexpr int kBookParts = 2;
+inline int book_blocks(int nbc) { return kBookParts + (nbc + 63) / 64; }
 
 // one block of a batched launch: scenario and block within it
 struct TileRef {
@@ -230,6 +238,7 @@ struct sw2d_handle {
     double *evapo = nullptr; int nevapo = 0; int evap_on = 0;
     double *Q = nullptr; int nq = 0, nst = 0; double dtoq = 1.0;
     int *src_r = nullptr, *src_c = nullptr;
+    double *src_rate = nullptr;         // 3 clock slots x nst x 2
     int storm_on = 0; sw2d_storm storm{};
     int ncls_on = 0; double ntab[sw2d::kMaxClasses] = {0};
     int out_r = -1, out_c = -1, out_edge = 0;
@@ -328,6 +337,9 @@ hipError_t launch_derive_f64(sw2d_handle *h, int field, double *out_dev, long fi
 hipError_t launch_derive_f32(sw2d_handle *h, int field, double *out_dev, long first, long count);
 hipError_t launch_derive_mix(sw2d_handle *h, int field, double *out_dev, long first, long count);
 hipError_t launch_peek(sw2d_handle *h, const StepCommon &sc);
+// the forcing of each descriptor's current iteration (clock slot s.slot_a)
+// into its clock, after the descriptors changed
+hipError_t launch_forcing(hipStream_t stream, const Scenario *scen, int n);
 int fused_waves_per_cu_f64(int features);  // resident one-wave blocks per CU
 int fused_waves_per_cu_f32(int features);
 int fused_waves_per_cu_mix(int features);

@@ -71,12 +71,12 @@ __device__ __forceinline__ double log_pos(double x)
 
 __device__ __forceinline__ double exp_d(double t)
 {
-    if (t != t) return t;
-    if (t > 709.0) return __longlong_as_double(0x7ff0000000000000LL);
-    if (t < -708.0) return 0.0;
-    double kd = floor(t * kInvLn2 + 0.5);
+    // without branches, so that several evaluations overlap: the series runs on
+    // t clamped to the range it holds for
+    const double x = __builtin_fmin(__builtin_fmax(t, -708.0), 709.0);
+    double kd = floor(x * kInvLn2 + 0.5);
     int k = (int)kd;
-    double r = (t - kd * kLn2Hi) - kd * kLn2Lo;
+    double r = (x - kd * kLn2Hi) - kd * kLn2Lo;
     double p = 1.0 / 6227020800.0;
     p = __builtin_fma(r, p, 1.0 / 479001600.0);
     p = __builtin_fma(r, p, 1.0 / 39916800.0);
@@ -93,7 +93,10 @@ __device__ __forceinline__ double exp_d(double t)
     int k1 = k / 2, k2 = k - k1;
     double s1 = __longlong_as_double((long long)((uint64_t)(k1 + 1023) << 52));
     double s2 = __longlong_as_double((long long)((uint64_t)(k2 + 1023) << 52));
-    return (er * s1) * s2;
+    double e = (er * s1) * s2;
+    e = t > 709.0 ? __longlong_as_double(0x7ff0000000000000LL) : e;
+    e = t < -708.0 ? 0.0 : e;
+    return t != t ? t : e;
 }
 
 __device__ __forceinline__ double log_d(double x)
