@@ -19,17 +19,15 @@ LIB = os.path.join(HERE, "libsw2d.so")
 DRIVER = os.path.join(HERE, "sw2d-efdc")
 
 # (source, extra flags); the FP32 kernel may fuse multiply-adds within one
-# source expression, nothing else may fuse any.  The fused kernels are
-# scheduled for instruction-level parallelism (LLVM's AMDGPU scheduler
-# strategies; the register counts, hence the waves per SIMD, stay as they
-# are): measured per launch on the 256-scenario batch and the 2048^2 storm,
-# "max-ilp" makes the FP32 form ~1% faster, "iterative-ilp" the FP64 and
-# mixed forms 0.3-2%.  Scheduling does not change what is rounded where.
-ILP_MAX = ["-mllvm", "-amdgpu-sched-strategy=max-ilp"]
+# source expression, nothing else may fuse any.  The FP64 fused kernel is
+# scheduled for instruction-level parallelism (one of LLVM's AMDGPU scheduler
+# strategies): one of 2048^2 125 against 127 us a launch.  The FP32 and mixed
+# forms gain nothing from it within the registers of five waves a SIMD.
+# Scheduling does not change what is rounded where.
 ILP_ITER = ["-mllvm", "-amdgpu-sched-strategy=iterative-ilp"]
 HIP_SOURCES = [("sw2d_api.hip", []), ("sw2d_fused64.hip", ILP_ITER),
-               ("sw2d_fused32.hip", ["-ffp-contract=on", *ILP_MAX]),
-               ("sw2d_fusedmix.hip", ["-ffp-contract=on", *ILP_ITER]), ("sw2d_plain.hip", []),
+               ("sw2d_fused32.hip", ["-ffp-contract=on"]),
+               ("sw2d_fusedmix.hip", ["-ffp-contract=on"]), ("sw2d_plain.hip", []),
                ("sw2d_batch.hip", []), ("sw2d_server.hip", []), ("sw2d_output.hip", []),
                ("sw2d_host.cpp", [])]
 DRIVER_SOURCES = ["sw2d_driver.cpp", "sw2d_io.cpp", "sw2d_efdc_config.cpp", "sw2d_gefdc.cpp", "sw2d_lorp.cpp"]

@@ -186,15 +186,18 @@ int flush_events(sw2d_handle *h)
     return SW2D_OK;
 }
 
+int device_cus(int device)
+{
+    int cus = 0;
+    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess) return 1;
+    return std::max(cus, 1);
+}
+
 // Resident one-wave blocks of the fused kernel over the device (waves per CU
 // at its register use x CUs): one "round" of a launch.
 long wave_slots(int device, int prec, int features)
 {
-    const int per_cu = fused_waves_per_cu(prec, features);
-    hipDeviceProp_t prop;
-    int cus = 0;
-    if (hipGetDeviceProperties(&prop, device) == hipSuccess) cus = prop.multiProcessorCount;
-    return (long)std::max(per_cu, 1) * std::max(cus, 1);
+    return (long)std::max(fused_waves_per_cu(prec, features), 1) * device_cus(device);
 }
 
 // blocks of one launch of a stand-alone grid at tile height H
@@ -225,19 +228,36 @@ std::vector<int> round_fill_heights(long slots, const std::function<long(int)> &
     return out;   // ascending
 }
 
-// Default tile height of the fused kernel (every tile is one wave): the
-// smallest height that fills whole rounds of wave slots, taking the fewest
-// rounds whose height is at most 48 (16 when none is).  sw2d_autotune replaces
-// it by a measured choice.
+// Default tile height of the fused kernel (every tile is one wave): the height
+// whose launch the model of the row loop finds shortest.  A tile of H rows is a
+// chain of H + 4.5 row times (six halo rows, three of them without fluxes), and a
+// row takes r + w units with w waves on the SIMD: the chip works through whole
+// rounds of wave slots at full occupancy and the rest of the tiles at the
+// occupancy they reach.  r from launches of 2048^2, 556 x 701 and 331 x 1009
+// grids at heights of 2 to 80 rows; the model orders those as measured.
+int model_tile_rows(int prec, long slots, long simds, const std::function<long(int)> &blocks)
+{
+    const double r = flux_bytes(prec) == 8 ? 2.1 : 3.3;
+    const double occ = (double)slots / simds;
+    int best = 2;
+    double best_t = INFINITY;
+    for (int H = 2; H <= 80; H++) {
+        const long n = blocks(H), rest = n % slots;
+        const double w = (double)((rest + simds - 1) / simds);
+        const double t = (H + 4.5) * ((double)(n / slots) * (r + occ) + (rest ? r + w : 0.0));
+        if (t < best_t) { best_t = t; best = H; }
+    }
+    return best;
+}
+
+// sw2d_autotune replaces it by a measured choice.
 int choose_tile_rows(const sw2d_handle *h)
 {
     if (h->prm.tile_rows > 0) return std::min(h->prm.tile_rows, 512);
-    const long slots = wave_slots(h->device, h->prm.precision,
-                                  features_of(make_common(const_cast<sw2d_handle *>(h))));
-    const std::vector<int> fit = round_fill_heights(slots, [&](int H) { return (long)blocks_at(h, H); });
-    for (auto it = fit.rbegin(); it != fit.rend(); ++it)
-        if (*it <= 48) return *it;
-    return 16;
+    const int feats = features_of(make_common(const_cast<sw2d_handle *>(h)));
+    const long slots = wave_slots(h->device, h->prm.precision, feats);
+    return model_tile_rows(h->prm.precision, slots, 4L * device_cus(h->device),
+                           [&](int H) { return (long)blocks_at(h, H); });
 }
 
 void set_tiles(sw2d_handle *h, int H)

@@ -171,6 +171,17 @@ __device__ __forceinline__ T face_flux(const u64 act, const TH ho, const TH hb, 
 
 constexpr int kMaxTileRows = 512;
 
+// Waves per SIMD that the registers have to leave room for.  Each of them issues
+// about one instruction in 5.5 cycles, so SIMDs are filled by more of them: a
+// row takes a wave (3.3 + w) units of time beside w - 1 others in the FP32 and
+// mixed forms, (2.1 + w) in FP64 (2048^2 and 331 x 1009 grids at w = 1 to 5).
+// 3 against 2 in FP64: 2048^2 134 -> 125 us, 24 grids of 128^2..1024^2 the same;
+// 5 against 4 in FP32: 2048^2 59.0 -> 56.8.  Six waves (80 registers) spill, and
+// so does the instantiation with every feature at these counts: 556 x 701 in
+// FP64, two waves a SIMD whatever its registers, 27.0 us without, 29.5 with.
+template <typename T, int F>
+constexpr int kMinWaves = (sizeof(T) == 8 ? 3 : 5) - ((F & kFeatSources) ? 1 : 0);
+
 // F: the features (kFeat*) this instantiation handles.  A feature missing
 // from F is compiled out (its uniforms, branches and loops), which the host
 // may only do for launches where no scenario uses it.  The arithmetic of
@@ -178,7 +189,7 @@ constexpr int kMaxTileRows = 512;
 // multiply-add, FP32 only within one source expression), so a scenario's
 // results do not depend on the instantiation that ran it.
 template <typename T, typename TH, int F>
-__global__ void __launch_bounds__(64)
+__global__ void __launch_bounds__(64, (kMinWaves<T, F>))
 fused_step(const Scenario *__restrict__ scen, const TileRef *__restrict__ tiles, const int nblocks,
            const int phase)
 {
@@ -280,6 +291,18 @@ fused_step(const Scenario *__restrict__ scen, const TileRef *__restrict__ tiles,
     const Arr<uint8_t> cls_in(map_on ? (const void *)d.cls : (const void *)d.z, map_on ? cells : 0u);
     __shared__ T nt_s[kMaxClasses];  // Manning coefficients of the classes
     if (kMap && lane < kMaxClasses) nt_s[lane] = (T)s.ntab[lane];
+    // FP64: the tables of the power in LDS.  Reads of them from memory share the
+    // counter of the row loads, and waiting for one of the former waits for the
+    // next row as well: four such waits a row with friction on both faces.  24
+    // grids of 128^2..1024^2 221 -> 195 us a launch, one of 2048^2 140 -> 134.
+    __shared__ double pow_s[kF32 ? 1 : 192];
+    const PowTablesLds ptab{pow_s};
+    if constexpr (!kF32) {
+        pow_s[lane] = kPowRecip[lane];
+        pow_s[64 + lane] = kPowNlog[lane];
+        pow_s[128 + lane] = kPowExp2[lane];
+        __syncthreads();
+    }
     const unsigned in1 = colin ? (unsigned)j : kOutside;
     const unsigned inT = colin ? (unsigned)j * (unsigned)sizeof(T) : kOutside;
     const unsigned inH = colin ? (unsigned)j * (unsigned)sizeof(TH) : kOutside;
@@ -477,7 +500,7 @@ fused_step(const Scenario *__restrict__ scen, const TileRef *__restrict__ tiles,
                 T ram = 0.00;
                 if (lanes(fr)) {
                     const T sqx = M::sqrt_(uu1_1 * uu1_1 + vva1 * vva1);
-                    ram = M::div_(gg * nf * nf * sqx, pow1333(hm1));
+                    ram = M::div_(gg * nf * nf * sqx, pow1333(hm1, ptab));
                 }
                 if constexpr (kF32) {
                     const T a = dt2half * ram;
@@ -513,7 +536,7 @@ fused_step(const Scenario *__restrict__ scen, const TileRef *__restrict__ tiles,
                 T ram = 0.00;
                 if (lanes(fr)) {
                     const T sqy = M::sqrt_(uua1 * uua1 + vv1_1 * vv1_1);
-                    ram = M::div_(gg * nf * nf * sqy, pow1333(hn1));
+                    ram = M::div_(gg * nf * nf * sqy, pow1333(hn1, ptab));
                 }
                 if constexpr (kF32) {
                     const T a = dt2half * ram;

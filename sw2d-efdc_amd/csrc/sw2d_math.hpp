@@ -113,14 +113,28 @@ static __constant__ const double kPowRecip[64] = {SW2D_POW_RECIP};
 static __constant__ const double kPowNlog[64] = {SW2D_POW_NLOG};
 static __constant__ const double kPowExp2[64] = {SW2D_POW_EXP2};
 
+// the tables where they lie, and a copy of them in LDS: recip, nlog, exp2 in a row
+struct PowTables {
+    __device__ __forceinline__ double recip(int i) const { return kPowRecip[i]; }
+    __device__ __forceinline__ double nlog(int i) const { return kPowNlog[i]; }
+    __device__ __forceinline__ double exp2(int i) const { return kPowExp2[i]; }
+};
+struct PowTablesLds {
+    const double *t;
+    __device__ __forceinline__ double recip(int i) const { return t[i]; }
+    __device__ __forceinline__ double nlog(int i) const { return t[64 + i]; }
+    __device__ __forceinline__ double exp2(int i) const { return t[128 + i]; }
+};
+
 // pow(x, 1.3333330) for 2^-700 <= x <= 2^500 (table-driven, see the top)
-__device__ __forceinline__ double pow1333_core(double x)
+template <typename Tab>
+__device__ __forceinline__ double pow1333_core(double x, const Tab &tab)
 {
     const uint64_t b = (uint64_t)__double_as_longlong(x);
     const int e = (int)(b >> 52) - 1023;
     const int i = (int)((b >> 46) & 63);
     const double m = __longlong_as_double((long long)((b & 0x000fffffffffffffULL) | 0x3ff0000000000000ULL));
-    const double r = __builtin_fma(m, kPowRecip[i], -1.0);
+    const double r = __builtin_fma(m, tab.recip(i), -1.0);
     double q = 1.0 / 7.0;
     q = __builtin_fma(r, q, -1.0 / 6.0);
     q = __builtin_fma(r, q, 1.0 / 5.0);
@@ -129,7 +143,7 @@ __device__ __forceinline__ double pow1333_core(double x)
     q = __builtin_fma(r, q, -0.5);
     const double lp = __builtin_fma(r * r, q, r);
     const double de = (double)e;
-    const double lx = __builtin_fma(de, kLn2Hi, __builtin_fma(de, kLn2Lo, kPowNlog[i] + lp));
+    const double lx = __builtin_fma(de, kLn2Hi, __builtin_fma(de, kLn2Lo, tab.nlog(i) + lp));
     const double t = kManningExp * lx;
     const double kd = __builtin_rint(t * (64.0 * kInvLn2));
     const int k = (int)kd;
@@ -141,14 +155,15 @@ __device__ __forceinline__ double pow1333_core(double x)
     p = __builtin_fma(rr, p, 1.0 / 6.0);
     p = __builtin_fma(rr, p, 0.5);
     const double P = __builtin_fma(rr * rr, p, rr);
-    const double T = kPowExp2[k & 63];
+    const double T = tab.exp2(k & 63);
     return __builtin_ldexp(__builtin_fma(T, P, T), k >> 6);
 }
 
 // pow(x, 1.3333330) for FP64
-__device__ __forceinline__ double pow1333(double x)
+template <typename Tab = PowTables>
+__device__ __forceinline__ double pow1333(double x, const Tab &tab = Tab())
 {
-    if (x >= 0x1p-700 && x <= 0x1p500) return pow1333_core(x);
+    if (x >= 0x1p-700 && x <= 0x1p500) return pow1333_core(x, tab);
     if (x != x) return x;
     if (!(x > 0.0)) return x == 0.0 ? 0.0 : __longlong_as_double(0x7ff8000000000000LL);
     if (x == __longlong_as_double(0x7ff0000000000000LL)) return x;
@@ -156,7 +171,8 @@ __device__ __forceinline__ double pow1333(double x)
 }
 
 // pow(x, 1.3333330) for FP32 (x > 0 on every path that uses the result)
-__device__ __forceinline__ float pow1333(float x)
+template <typename Tab>
+__device__ __forceinline__ float pow1333(float x, const Tab &)
 {
     return __builtin_amdgcn_exp2f((float)kManningExp * __builtin_amdgcn_logf(x));
 }
