@@ -29,18 +29,21 @@
 // barriers: each wave is independent.  The grid is one wave per tile plus the
 // bookkeeping waves.
 //
-// What bounds it: issue of vector instructions (FP32 and mixed forms), the
-// latency of chains of FP64 operations at two waves per SIMD (FP64 form).  So
-// the row is written for few vector instructions: the conditions are lane
-// masks on the scalar unit, rows are addressed by a scalar offset, each
-// upwind product is formed once (the south one of a row is the north one of
-// the next, the east one of a cell the west one of its east neighbour), the
-// weirs, the momentum update and the first continuity run only in rows where
-// a lane needs them, and a row without fluxes and sources keeps its depths.
-// Measured per launch against per-lane booleans and every product formed
-// twice, results equal bit for bit: 48 grids of 128^2..1024^2 in FP32 145 ->
-// 121 us, 24 of them in FP64 217 -> 197 us; one 2048^2 grid FP32 91 -> 79,
-// FP64 161 -> 146 us.
+// What bounds it: the number of instructions, scalar ones as much as vector ones
+// (a wave issues one in 4 to 5 cycles whatever its dependencies, and the waves of
+// a SIMD get in each other's way), and on states past the 256 MB cache the loads
+// in flight.  So the row is written for few instructions: the conditions are lane
+// masks on the scalar unit, each upwind product is formed once (the south one of a
+// row is the north one of the next, the east one of a cell the west one of its
+// east neighbour), the weirs, the momentum update and the first continuity run
+// only in rows where a lane needs them, a row without fluxes and sources keeps its
+// depths, what changes only at the first or last rows of a tile (rows outside the
+// grid, rows before the first output) is set there and not tested in every row,
+// and the three rows above a tile run in a short loop of their own.  Measured per
+// launch against per-row tests, selects and resources, and with the FP64 power's
+// coefficients from LDS, same results: one 2048^2 grid FP32 57.8 -> 51.2 us, FP64
+// 127 -> 118; 1537 x 2311 mixed 54.5 -> 47.2; 331 x 1009 FP32 17.5 -> 16.1; 256^2
+// FP64 13.2 -> 12.1; 24 grids of 128^2..1024^2 FP64 158 -> 144.
 //
 // T is the type of the fluxes and of the momentum arithmetic, TH that of the
 // depths, the continuity updates and every switch that tests a depth.
@@ -66,6 +69,16 @@ typedef unsigned long long u64;
 __device__ __forceinline__ u64 vote(bool p) { return __builtin_amdgcn_ballot_w64(p); }
 __device__ __forceinline__ bool lanes(u64 m) { return __builtin_amdgcn_inverse_ballot_w64(m); }
 
+// 1 for a mask with a lane in it, else 0, on the scalar unit
+__device__ __forceinline__ unsigned any_lane(u64 m)
+{
+    unsigned n;
+    asm("s_bcnt1_i32_b64 %0, %1" : "=s"(n) : "s"(m) : "scc");
+    return n < 1u ? n : 1u;
+}
+// a wave-uniform condition that the compiler cannot see to be uniform
+__device__ __forceinline__ bool uniform(bool p) { return __builtin_amdgcn_readfirstlane((int)p) != 0; }
+
 // One scenario array, read and written through a buffer resource (base and
 // range in scalar registers): a lane's byte offset within the row stays in one
 // register for the whole tile and the row's byte offset is scalar, so a row
@@ -80,32 +93,29 @@ template <typename V> struct Arr {
     unsigned bytes;
     __device__ Arr(const void *q, unsigned cells)
         : p(const_cast<void *>(q)), bytes(cells * (unsigned)sizeof(V)) {}
-    // the resource for one row; on == false: an empty range, so that the row
-    // reads ghosts (its stores are dropped) without a branch around the access:
-    // a branch would make the count of accesses in flight unknown, and the
-    // next row's wait would cover the prefetched row as well.  0x00020000: the
-    // 32-bit data format (a buffer with the invalid format reads zeros)
-    __device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc(bool on) const
+    // 0x00020000: the 32-bit data format (a buffer with the invalid format reads
+    // zeros)
+    __device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc() const
     {
-        return __builtin_amdgcn_make_buffer_rsrc(p, (short)0, on ? bytes : 0u, 0x00020000);
+        return __builtin_amdgcn_make_buffer_rsrc(p, (short)0, bytes, 0x00020000);
     }
-    __device__ __forceinline__ V load(unsigned off, unsigned row, bool on) const
+    __device__ __forceinline__ V load(unsigned off, unsigned row) const
     {
         const unsigned ro = row * (unsigned)sizeof(V);
         if constexpr (sizeof(V) == 1)
-            return __builtin_amdgcn_raw_buffer_load_b8(rsrc(on), (int)off, (int)ro, 0);
+            return __builtin_amdgcn_raw_buffer_load_b8(rsrc(), (int)off, (int)ro, 0);
         else if constexpr (sizeof(V) == 4)
-            return __builtin_bit_cast(V, __builtin_amdgcn_raw_buffer_load_b32(rsrc(on), (int)off, (int)ro, 0));
+            return __builtin_bit_cast(V, __builtin_amdgcn_raw_buffer_load_b32(rsrc(), (int)off, (int)ro, 0));
         else
-            return __builtin_bit_cast(V, __builtin_amdgcn_raw_buffer_load_b64(rsrc(on), (int)off, (int)ro, 0));
+            return __builtin_bit_cast(V, __builtin_amdgcn_raw_buffer_load_b64(rsrc(), (int)off, (int)ro, 0));
     }
-    __device__ __forceinline__ void store(unsigned off, unsigned row, V v, bool on) const
+    __device__ __forceinline__ void store(unsigned off, unsigned row, V v) const
     {
         const unsigned ro = row * (unsigned)sizeof(V);
         if constexpr (sizeof(V) == 4)
-            __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, v), rsrc(on), (int)off, (int)ro, 0);
+            __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, v), rsrc(), (int)off, (int)ro, 0);
         else
-            __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, v), rsrc(on), (int)off, (int)ro, 0);
+            __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, v), rsrc(), (int)off, (int)ro, 0);
     }
 };
 
@@ -167,6 +177,16 @@ __device__ __forceinline__ T face_flux(const u64 act, const TH ho, const TH hb, 
         val = lanes(B4) ? up : val;
     }
     return val;
+}
+
+// the tables of the power, to be read anew at each use
+template <typename T>
+__device__ __forceinline__ PowTablesLds pow_tables(const double *t)
+{
+    if constexpr (sizeof(T) == 4) return PowTablesLds{t, 0};
+    int zero;
+    asm volatile("v_mov_b32 %0, 0" : "=v"(zero));
+    return PowTablesLds{t, zero};
 }
 
 constexpr int kMaxTileRows = 512;
@@ -266,9 +286,8 @@ fused_step(const Scenario *__restrict__ scen, const TileRef *__restrict__ tiles,
     const int R = s.R, C = s.C, P = d.P;
     const int j0 = strip * d.W;
     const int j = j0 - 3 + lane;
-    const bool colin = (j >= 0) && (j < C);
     const bool colout = (lane >= 3) && (lane < 3 + d.W) && (j < C);
-    const u64 in_cols = vote(colin), out_cols = vote(colout);
+    const u64 out_cols = vote(colout);
     const int r0 = chunk * d.H;
     const int r1 = (r0 + d.H < R) ? r0 + d.H : R;
 
@@ -295,36 +314,52 @@ fused_step(const Scenario *__restrict__ scen, const TileRef *__restrict__ tiles,
     // counter of the row loads, and waiting for one of the former waits for the
     // next row as well: four such waits a row with friction on both faces.  24
     // grids of 128^2..1024^2 221 -> 195 us a launch, one of 2048^2 140 -> 134.
-    __shared__ double pow_s[kF32 ? 1 : 192];
-    const PowTablesLds ptab{pow_s};
+    __shared__ double pow_s[kF32 ? 2 : kPowLds];
     if constexpr (!kF32) {
         pow_s[lane] = kPowRecip[lane];
         pow_s[64 + lane] = kPowNlog[lane];
         pow_s[128 + lane] = kPowExp2[lane];
+        if (lane < 16) pow_s[192 + lane] = kPowCoefMem[lane];
         __syncthreads();
     }
-    const unsigned in1 = colin ? (unsigned)j : kOutside;
-    const unsigned inT = colin ? (unsigned)j * (unsigned)sizeof(T) : kOutside;
-    const unsigned inH = colin ? (unsigned)j * (unsigned)sizeof(TH) : kOutside;
-    const unsigned in8 = colin ? (unsigned)j * 8u : kOutside;
-    const unsigned outT = colout ? (unsigned)j * (unsigned)sizeof(T) : kOutside;
-    const unsigned outH = colout ? (unsigned)j * (unsigned)sizeof(TH) : kOutside;
-    const int kbeg = r0 - 3, kend = r1 + 3;
+    const int kbeg = r0 - 3, kend = r1 + 3, kload = kend < R ? kend : R;
+    // Row to load next: its offset (in elements), and the lanes' byte offsets.
+    // While that row is outside the grid (or past the last one that is needed)
+    // every lane's offset is kOutside, so it reads ghosts; a branch around the
+    // loads would make the count of accesses in flight unknown, and the next
+    // row's wait would cover the prefetched row as well.  aim() sets them for
+    // row k; it is called where they change (row kaim) and nowhere else.
+    unsigned offT, offH, off8, off1, row_in = 0, row_step;
+    u64 cols_n;  // lanes inside the grid in that row
+    int kaim;
+    auto aim = [&](const int k) {
+        const bool on = k >= 0 && k < kload;
+        int c = j;
+        asm volatile("" : "+v"(c));  // computed here: not held in registers
+        const bool in = on && c >= 0 && c < C;
+        offT = in ? (unsigned)c * (unsigned)sizeof(T) : kOutside;
+        offH = in ? (unsigned)c * (unsigned)sizeof(TH) : kOutside;
+        off8 = in ? (unsigned)c * 8u : kOutside;
+        off1 = in ? (unsigned)c : kOutside;
+        cols_n = vote(in);
+        row_in = on ? (unsigned)k * (unsigned)P : 0u;
+        row_step = on ? (unsigned)P : 0u;
+        kaim = k < 0 ? 0 : k < kload ? kload : 0x7fffffff;
+    };
     TH nh;
     T nu, nv;
     double nz;
     uint8_t ncl;
-    auto load_row = [&](int k) {
-        const bool on = k >= 0 && k < R;
-        const unsigned row = on ? (unsigned)k * (unsigned)P : 0u;
-        nh = h_in.load(inH, row, on);
-        nu = um_in.load(inT, row, on);
-        nv = vn_in.load(inT, row, on);
-        nz = zg.load(in8, row, on);
-        if constexpr (kMap) ncl = cls_in.load(in1, row, on);
+    auto load_row = [&]() {
+        nh = h_in.load(offH, row_in);
+        nu = um_in.load(offT, row_in);
+        nv = vn_in.load(offT, row_in);
+        nz = zg.load(off8, row_in);
+        if constexpr (kMap) ncl = cls_in.load(off1, row_in);
         else ncl = 0;
     };
-    load_row(kbeg);
+    aim(kbeg);
+    load_row();
 
     // CFL candidates only for an adaptive time step; a wave-uniform flag, so
     // a scenario runs the same instructions alone and in a mixed batch
@@ -342,15 +377,15 @@ fused_step(const Scenario *__restrict__ scen, const TileRef *__restrict__ tiles,
         if (!vote(here)) nst = 0;
     }
     const double *src_rate = s.src_rate + (size_t)it.slot_a * 2 * s.nst;
-    const T gg = (T)s.g, dx = (T)s.dx, dy = (T)s.dy;
+    const T gg = (T)s.g, dx = (T)s.dx;  // cells are square: dy = dx
     const TH thh = (TH)s.th;
-    const T rdx = (T)(1.0 / s.dx), rdy = (T)(1.0 / s.dy);
+    const T rdx = (T)(1.0 / s.dx);
     const T dt2 = (T)st.dt2;
     const TH dt2h = (TH)st.dt2;
-    const T dt2dx = (T)(st.dt2 / s.dx), dt2dy = (T)(st.dt2 / s.dy);
+    const T dt2dx = (T)(st.dt2 / s.dx);
     // FP32 momentum: the upwind differences carry sums of two face
-    // velocities, so dt2/dx and dt2/dy enter with the two halvings folded
-    const T dt2dx4 = T(0.25) * dt2dx, dt2dy4 = T(0.25) * dt2dy, dt2half = T(0.5) * dt2;
+    // velocities, so dt2/dx enters with the two halvings folded
+    const T dt2dx4 = T(0.25) * dt2dx, dt2half = T(0.5) * dt2;
     const T rn = (T)s.rn;
 
     // forcing of this iteration: first continuity at t, second at t + dt
@@ -382,7 +417,10 @@ fused_step(const Scenario *__restrict__ scen, const TileRef *__restrict__ tiles,
     const TH ewl = (TH)s.EV_WL_min;
     // no water is added or taken in the second continuity: a row without
     // fluxes then keeps its depths
-    const bool calm2 = !storm_on && nst == 0 && rr2 == 0.0 && ev2 == 0.0;
+    const bool calm2 = uniform(!storm_on && nst == 0 && rr2 == 0.0 && ev2 == 0.0);
+    // one forcing for all depths (no evaporation, the same fraction of the rain)
+    const bool even = uniform(s.P_lake == s.P_land && ev1 == 0.0 && ev2 == 0.0);
+    const int out_edge = __builtin_amdgcn_readfirstlane(s.out_edge);
 
     // the outlet's row, where its column is among this wave's lanes, and its lane
     const int ol = s.out_edge ? s.out_c - (j0 - 3) : -1;
@@ -401,43 +439,100 @@ fused_step(const Scenario *__restrict__ scen, const TileRef *__restrict__ tiles,
     T dzn1 = 0, dzw1 = 0;  // FP32 form: z(k-2) - z(k-1) and z(k-1, j-1) - z(k-1, j)
     T nc1 = rn, nc2 = rn;
     T umnP = 0, vnnP = 0, umpP = 0, vnpP = 0;
-    // faces that may carry flux: rows k-1, k-2, k-3 (north), k-2, k-3 (west)
-    u64 FXP = 0, FXQ = 0, FYP = 0, FYQ = 0;
+    // rows with faces that may carry flux: bit 0 north faces, bit 1 west faces of
+    // row k-1, bits 2 and 3 of row k-2, and so on
+    unsigned flow = 0;
+    unsigned outT = kOutside, outH = kOutside, row_out = 0;  // of the next row to store
+    const int kcfl = adapt ? r1 : -1000;
     u64 D1 = 0;  // cells of row k-3 that dried in the first continuity
+    T div1 = 0;  // its flux divergence of row k-3, and which fluxes of it were taken out
+    unsigned cut1 = 0;
 
+    // sums over all lanes; those outside the output columns are dropped at the end
     double acc_vol = 0, acc_src = 0, acc_clip = 0;
     // CFL: the largest |u| + sqrt(g h) per direction; min_f dx / s_f = dx / max_f s_f
     // because rounding dx / s is monotone in s
     T smax_x = 0, smax_y = 0;
 
-    // everything loaded so far is here (vmcnt, lgkmcnt 0): the loop's own waits
-    // then count only its own accesses
-    __builtin_amdgcn_s_waitcnt(0x0070);
-    for (int k = kbeg; k < kend; ++k) {
-        const TH h0 = nh;
-        const T u0 = nu, v0 = nv;
-        const double z0 = nz;
-        const uint8_t cl0 = ncl;
-        load_row(k + 1);
-        // FP32 form: z0 holds the bed steps of row k's cell to its north (low
+    // row k: what the rows after it need of it
+    struct Front {
+        TH h, hm, hn;
+        T u, v, uu1, uu1w, vv1, px, py, dzn, dzw, nc;
+        double z;
+        u64 A, W, L;
+    };
+    auto front = [&](const int k) __attribute__((always_inline)) -> Front {
+        Front o;
+        o.h = nh; o.u = nu; o.v = nv; o.z = nz;
+        const uint8_t cl = ncl;
+        const u64 cols = cols_n;
+        row_in += row_step;
+        if (k + 1 == kaim) aim(k + 1);
+        load_row();
+        // FP32 form: z holds the bed steps of row k's cell to its north (low
         // word) and west (high word) neighbours, NaN for an inactive cell
-        const u32x2 zsteps = __builtin_bit_cast(u32x2, z0);
-        const T dzn0 = (T)__uint_as_float(zsteps.x), dzw0 = (T)__uint_as_float(zsteps.y);
-        const u64 A0 = vote(kH32 ? (dzw0 == dzw0) : (z0 == z0)) & (k >= 0 && k < R ? in_cols : 0ull);
-        const u64 W0 = vote(h0 > thh), L0 = vote(h0 < thh);
-        T nc0 = rn;
-        if constexpr (kMap) nc0 = map_on ? nt_s[cl0] : rn;
+        const u32x2 zsteps = __builtin_bit_cast(u32x2, o.z);
+        o.dzn = (T)__uint_as_float(zsteps.x);
+        o.dzw = (T)__uint_as_float(zsteps.y);
+        o.A = vote(kH32 ? (o.dzw == o.dzw) : (o.z == o.z)) & cols;
+        o.W = vote(o.h > thh);
+        o.L = vote(o.h < thh);
+        o.nc = rn;
+        if constexpr (kMap) o.nc = map_on ? nt_s[cl] : rn;
 
-        // ---- row k: face depths and velocities (hm_hn, uu1_vv1) ----
+        // ---- face depths and velocities (hm_hn, uu1_vv1) ----
         // (row 0's north and column 0's west faces carry no flux, so their
         // velocities are 0 whatever the face depth)
-        const TH hn0d = TH(0.50) * (h0 + from_west(h0));
-        const TH hm0d = TH(0.50) * (h0 + h1);
-        const T hn0 = (T)hn0d, hm0 = (T)hm0d;
-        const T uu1_0 = (hm0d >= thh) ? M::div_(u0, hm0) : T(0.00);
-        const T vv1_0 = (hn0d >= thh) ? M::div_(v0, hn0) : T(0.0);
+        o.hn = TH(0.50) * (o.h + from_west(o.h));
+        o.hm = TH(0.50) * (o.h + h1);
+        o.uu1 = (o.hm >= thh) ? M::div_(o.u, (T)o.hm) : T(0.00);
+        o.vv1 = (o.hn >= thh) ? M::div_(o.v, (T)o.hn) : T(0.0);
 
-        if (adapt && k >= r0 && k < r1) {
+        // upwind products of the convection terms between rows k-1 and k: the
+        // south one of row k-1 and the north one of row k, so each is formed
+        // once and carried.  FP32: without the halvings (see dt2dx4)
+        o.uu1w = from_west(o.uu1);
+        if constexpr (kF32) {
+            const T sr = o.uu1 + uu1_1;
+            o.px = sr * (o.u + u1) + M::abs_(sr) * (u1 - o.u);
+            const T sa = o.uu1 + o.uu1w;
+            o.py = sa * (o.v + v1) + M::abs_(sa) * (v1 - o.v);
+        } else {
+            const T ur = T(0.50) * (o.uu1 + uu1_1);
+            o.px = ur * (o.u + u1) * T(0.50) + M::abs_(ur) * (u1 - o.u) * T(0.50);
+            const T av = T(0.50) * (o.uu1 + o.uu1w);
+            o.py = av * (o.v + v1) * T(0.50) + M::abs_(av) * (v1 - o.v) * T(0.50);
+        }
+        return o;
+    };
+    auto push = [&](const Front &o) __attribute__((always_inline)) {
+        h3 = h2; h2 = h1; h1 = o.h;
+        z2 = z1; z1 = o.z;
+        A3 = A2; A2 = A1; A1 = o.A;
+        W2 = W1; W1 = o.W;
+        L2 = L1; L1 = o.L;
+        u1 = o.u; v1 = o.v;
+        uu1_1 = o.uu1;
+        vv1_2 = vv1_1; vv1_1 = o.vv1;
+        px1 = o.px; py1 = o.py;
+        dzn1 = o.dzn; dzw1 = o.dzw;
+        nc2 = nc1; nc1 = o.nc;
+    };
+
+    // the three rows above feed the window only
+    for (int k = kbeg; k < r0; ++k) push(front(k));
+    // everything loaded so far is here (vmcnt, lgkmcnt 0): the loop's own waits
+    // then count only its own accesses (a wait for a load from before it would
+    // be a wait for the stores of the row before in every later row)
+    __builtin_amdgcn_s_waitcnt(0x0070);
+    for (int k = r0; k < kend; ++k) {
+        const Front o = front(k);
+        const TH hm0d = o.hm, hn0d = o.hn;
+        const T hm0 = (T)hm0d, hn0 = (T)hn0d, uu1_0 = o.uu1, vv1_0 = o.vv1, px0 = o.px, py0 = o.py;
+        const T uu1_0w = o.uu1w;
+        const u64 A0 = o.A;
+
+        if (k < kcfl) {
             // CFL candidates of the incoming state on the faces of row k
             if (lanes(A0 & A1 & out_cols & vote(hm0d > thh))) {
                 const T w = M::abs_(uu1_0) + M::sqrt_(gg * hm0);
@@ -449,32 +544,16 @@ fused_step(const Scenario *__restrict__ scen, const TileRef *__restrict__ tiles,
             }
         }
 
-        // upwind products of the convection terms between rows f = k-1 and k:
-        // the south one of row f and the north one of row f + 1, so each is
-        // formed once and carried.  FP32: without the halvings (see dt2dx4)
-        const T uu1_0w = from_west(uu1_0);
-        T px0, py0;
-        if constexpr (kF32) {
-            const T sr = uu1_0 + uu1_1;
-            px0 = sr * (u0 + u1) + M::abs_(sr) * (u1 - u0);
-            const T sa = uu1_0 + uu1_0w;
-            py0 = sa * (v0 + v1) + M::abs_(sa) * (v1 - v0);
-        } else {
-            const T ur = T(0.50) * (uu1_0 + uu1_1);
-            px0 = ur * (u0 + u1) * T(0.50) + M::abs_(ur) * (u1 - u0) * T(0.50);
-            const T av = T(0.50) * (uu1_0 + uu1_0w);
-            py0 = av * (v0 + v1) * T(0.50) + M::abs_(av) * (v1 - v0) * T(0.50);
-        }
-
         // ---- fluxes of row f = k-1 (flux, SW2D-EFDC.cu:97-353) ----
         const int f = k - 1;
         T umn = 0, vnn = 0;
-        // rows before r0 - 1 feed no output row: the warm-up only builds the window
         // x direction: um at the north face of (f, j); w = row f-1, e = row f
         // y direction: vn at the west face of (f, j); s = column j-1, n = column j
-        const u64 FX = k >= r0 ? A1 & A2 & (W1 | W2) : 0ull;
-        const u64 FY = (k >= r0 && k <= r1 + 1) ? A1 & (A1 << 1) & (W1 | (W1 << 1)) : 0ull;
+        const u64 FX = A1 & A2 & (W1 | W2);
+        const u64 FY = A1 & (A1 << 1) & (W1 | (W1 << 1));
+        flow <<= 2;
         if (FX) {
+            flow |= 1u;
             umn = face_flux<T, TH>(FX, h1, h2, dzn1, z1, z2, W1, W2, L1, L2, thh, gg,
                                    [&](const T hm1, const T dsurf, const u64 fr) {
                 const T u13 = gg * hm1 * dt2dx * dsurf;
@@ -486,21 +565,21 @@ fused_step(const Scenario *__restrict__ scen, const TileRef *__restrict__ tiles,
                     const T sd = vv1_1 + vv1_2;
                     pd = sd * (u1w + u1) + M::abs_(sd) * (u1w - u1);
                     u11 = dt2dx4 * (px0 - px1);
-                    u12 = dt2dy4 * (from_east(pd) - pd);
+                    u12 = dt2dx4 * (from_east(pd) - pd);
                 } else {
                     const T vd = T(0.50) * (vv1_1 + vv1_2);
                     pd = vd * (u1w + u1) * T(0.50) + M::abs_(vd) * (u1w - u1) * T(0.50);
                     u11 = dt2dx * (px0 - px1);
-                    u12 = dt2dy * (from_east(pd) - pd);
+                    u12 = dt2dx * (from_east(pd) - pd);
                 }
                 u12 = (j != 0) ? u12 : T(0);
                 // uua_vva (489-522): vva of row f
                 const T vva1 = T(0.250) * (vv1_1 + from_east(vv1_1) + vv1_2 + from_east(vv1_2));
-                const T nf = map_on ? T(0.5) * (nc2 + nc1) : rn;
+                const T nf = kMap ? T(0.5) * (nc2 + nc1) : rn;  // rn itself without a map
                 T ram = 0.00;
                 if (lanes(fr)) {
                     const T sqx = M::sqrt_(uu1_1 * uu1_1 + vva1 * vva1);
-                    ram = M::div_(gg * nf * nf * sqx, pow1333(hm1, ptab));
+                    ram = M::div_(gg * nf * nf * sqx, pow1333(hm1, pow_tables<T>(pow_s)));
                 }
                 if constexpr (kF32) {
                     const T a = dt2half * ram;
@@ -511,32 +590,33 @@ fused_step(const Scenario *__restrict__ scen, const TileRef *__restrict__ tiles,
                 }
             });
         }
-        if (FY) {
+        if (FY && k < r1 + 2) {
+            flow |= 2u;
             vnn = face_flux<T, TH>(FY, h1, from_west(h1), dzw1, z1, kH32 ? 0.0 : from_west(z1), W1,
                                    W1 << 1, L1, L1 << 1, thh, gg,
                                    [&](const T hn1, const T dsurf, const u64 fr) {
-                const T v13 = gg * hn1 * dt2dy * dsurf;
+                const T v13 = gg * hn1 * dt2dx * dsurf;
                 const T v1w = from_west(v1), uu1_1w = from_west(uu1_1);
                 T v11, v12, pd;
                 if constexpr (kF32) {
                     const T sq = vv1_1 + from_west(vv1_1);
                     pd = sq * (v1w + v1) + M::abs_(sq) * (v1w - v1);
                     v11 = dt2dx4 * (py0 - py1);
-                    v12 = dt2dy4 * (from_east(pd) - pd);
+                    v12 = dt2dx4 * (from_east(pd) - pd);
                 } else {
                     const T qv = T(0.50) * (vv1_1 + from_west(vv1_1));
                     pd = qv * (v1w + v1) * T(0.50) + M::abs_(qv) * (v1w - v1) * T(0.50);
                     v11 = dt2dx * (py0 - py1);
-                    v12 = dt2dy * (from_east(pd) - pd);
+                    v12 = dt2dx * (from_east(pd) - pd);
                 }
                 v11 = (f != 0) ? v11 : T(0);
                 // uua_vva (489-522): uua of row f
                 const T uua1 = T(0.250) * (uu1_1 + uu1_0 + uu1_1w + uu1_0w);
-                const T nf = map_on ? T(0.5) * (from_west(nc1) + nc1) : rn;
+                const T nf = kMap ? T(0.5) * (from_west(nc1) + nc1) : rn;
                 T ram = 0.00;
                 if (lanes(fr)) {
                     const T sqy = M::sqrt_(uua1 * uua1 + vv1_1 * vv1_1);
-                    ram = M::div_(gg * nf * nf * sqy, pow1333(hn1, ptab));
+                    ram = M::div_(gg * nf * nf * sqy, pow1333(hn1, pow_tables<T>(pow_s)));
                 }
                 if constexpr (kF32) {
                     const T a = dt2half * ram;
@@ -553,15 +633,18 @@ fused_step(const Scenario *__restrict__ scen, const TileRef *__restrict__ tiles,
         // the next row's north ones) carry nothing skip it
         const int g = k - 2;
         u64 D0 = 0;
-        T umpg = umnP, vnpg = vnnP;
-        if (k >= r0 + 1 && ((FX | FXP | FYP) || g == orow)) {
-            const bool wet = h2 > ewl;
-            const T Pc = wet ? P_lake : P_land;
-            const T E = wet ? ev1t : T(0.000);
+        T umpg = umnP, vnpg = vnnP, div0 = 0;
+        unsigned cut = 0;  // fluxes of row g taken out: bit 0 north faces, bit 1 west faces
+        if ((flow & 13u) || g == orow) {
+            T Pc = P_land, E = T(0.000);
+            if (!even) {
+                const bool wet = h2 > ewl;
+                Pc = wet ? P_lake : P_land;
+                E = wet ? ev1t : T(0.000);
+            }
             T rr = rr1t;
             if (storm_on) {
-                const int gi = g - (r0 - 5);
-                const T gy = gy_s[0][gi < 0 ? 0 : gi];
+                const T gy = gy_s[0][g - (r0 - 5)];
                 if constexpr (kF32) rr = pk1 * gy;
                 else rr = storm1 ? (T)(s.st_peak * (gx1 * gy)) : T(0);
             }
@@ -575,37 +658,43 @@ fused_step(const Scenario *__restrict__ scen, const TileRef *__restrict__ tiles,
                 qo_eff = (h2 > thh) ? T(0.5440) * h2t * M::sqrt_(gg * h2t) : T(0);
                 const T du1 = qo_eff - umnP, du2 = umn - (-qo_eff);
                 const T dv3 = vnnPe - (-qo_eff), dv4 = qo_eff - vnnP;
-                if (s.out_edge <= 2) du = lanes(out_lane) ? (s.out_edge == 1 ? du1 : du2) : du;
-                else dv = lanes(out_lane) ? (s.out_edge == 3 ? dv3 : dv4) : dv;
+                if (out_edge <= 2) du = lanes(out_lane) ? (out_edge == 1 ? du1 : du2) : du;
+                else dv = lanes(out_lane) ? (out_edge == 3 ? dv3 : dv4) : dv;
             }
-            const T rhs = M::divc_(du, dx, rdx) + M::divc_(dv, dy, rdy) - ql -
-                          rr * Pc + E;
+            div0 = M::divc_(du, dx, rdx) + M::divc_(dv, dx, rdx);
+            const T rhs = div0 - ql - rr * Pc + E;
             const TH hr = h2 - dt2h * (TH)rhs;
             D0 = vote(MH::max_(hr, TH(0.00)) < thh) & A2;
             // ---- treat_error on the faces of row g (695-725) ----
             if (D0 | D1) {
-                umpg = lanes((D1 & vote(umnP > 0)) | (D0 & vote(umnP < 0))) ? T(0) : umnP;
-                vnpg = lanes(((D0 << 1) & vote(vnnP > 0)) | (D0 & vote(vnnP < 0))) ? T(0) : vnnP;
+                const u64 zx = (D1 & vote(umnP > 0)) | (D0 & vote(umnP < 0));
+                const u64 zy = ((D0 << 1) & vote(vnnP > 0)) | (D0 & vote(vnnP < 0));
+                if (zx | zy) {
+                    umpg = lanes(zx) ? T(0) : umnP;
+                    vnpg = lanes(zy) ? T(0) : vnnP;
+                    cut = any_lane(zx) | any_lane(zy) << 1;
+                }
                 if (g == orow) qo_eff = lanes(D0) ? T(0) : qo_eff;
             }
         }
 
         // ---- second continuity of row q = k-3 at time t + dt; store ----
         const int q = k - 3;
-        const bool put = k >= r0 + 3;
         TH h2v = 0;
-        if (put) {
-            if (calm2 && !(FXP | FXQ | FYQ) && q != orow && !vote(!(h3 >= TH(0)))) {
+        if (k >= r0 + 3) {
+            if (calm2 && !(flow & 52u) && q != orow && !vote(!(h3 >= TH(0)))) {
                 h2v = lanes(A3) ? h3 : TH(0);
-                if (lanes(A3 & out_cols)) acc_vol += (double)h2v;
+                acc_vol += (double)h2v;
             } else {
-                const bool wet = h3 > ewl;
-                const T Pc = wet ? P_lake : P_land;
-                const T E = wet ? ev2t : T(0.000);
+                T Pc = P_land, E = T(0.000);
+                if (!even) {
+                    const bool wet = h3 > ewl;
+                    Pc = wet ? P_lake : P_land;
+                    E = wet ? ev2t : T(0.000);
+                }
                 T rr = rr2t;
                 if (storm_on) {
-                    const int qi = q - (r0 - 6);
-                    const T gy = gy_s[1][qi < 0 ? 0 : qi];
+                    const T gy = gy_s[1][q - (r0 - 6)];
                     if constexpr (kF32) rr = pk2 * gy;
                     else rr = storm2 ? (T)(s.st_peak * (gx2 * gy)) : T(0);
                 }
@@ -613,17 +702,22 @@ fused_step(const Scenario *__restrict__ scen, const TileRef *__restrict__ tiles,
                 for (int i = 0; i < nst; ++i)
                     if (s.src_r[i] == q && s.src_c[i] == j)
                         ql = (T)(adapt ? source_rate(s, i, st.tm) : src_rate[2 * i + 1]);
-                const T vnpPe = from_east(vnpP);
-                T du = umpg - umpP, dv = vnpPe - vnpP;
-                if (q == orow) {
-                    const T du1 = qo_eff - umpP, du2 = umpg - (-qo_eff);
-                    const T dv3 = vnpPe - (-qo_eff), dv4 = qo_eff - vnpP;
-                    if (s.out_edge <= 2) du = lanes(out_lane) ? (s.out_edge == 1 ? du1 : du2) : du;
-                    else dv = lanes(out_lane) ? (s.out_edge == 3 ? dv3 : dv4) : dv;
+                // FP64: the divergence is the first continuity's where treat_error
+                // left the row's fluxes as they were (two divisions less; in FP32
+                // forming it anew costs less than the test)
+                T div = div1;
+                if (kF32 || (cut1 | (cut & 1u)) || q == orow) {
+                    const T vnpPe = from_east(vnpP);
+                    T du = umpg - umpP, dv = vnpPe - vnpP;
+                    if (q == orow) {
+                        const T du1 = qo_eff - umpP, du2 = umpg - (-qo_eff);
+                        const T dv3 = vnpPe - (-qo_eff), dv4 = qo_eff - vnpP;
+                        if (out_edge <= 2) du = lanes(out_lane) ? (out_edge == 1 ? du1 : du2) : du;
+                        else dv = lanes(out_lane) ? (out_edge == 3 ? dv3 : dv4) : dv;
+                    }
+                    div = M::divc_(du, dx, rdx) + M::divc_(dv, dx, rdx);
                 }
-                const T rhs = M::divc_(du, dx, rdx) + M::divc_(dv, dy, rdy) - ql -
-                              rr * Pc + E;
-                const u64 sum = A3 & out_cols;
+                const T rhs = div - ql - rr * Pc + E;
                 if constexpr (kH32) {
                     // FP32 form: the depth update h3 - dt2 rhs is rounded
                     // stochastically.  TwoSum gives the exact rounding error er of
@@ -650,53 +744,54 @@ fused_step(const Scenario *__restrict__ scen, const TileRef *__restrict__ tiles,
                     // (exact: 48 bits suffice) is needed only then
                     const u64 neg = vote(sm <= T(0)) & (vote(sm < T(0)) | vote(er < T(0)));
                     if (neg) {
-                        if (lanes(neg & sum)) acc_clip += -((double)sm + (double)er);
+                        if (lanes(neg & A3)) acc_clip += -((double)sm + (double)er);
                         h2v = lanes(neg) ? TH(0) : h2v;
                     }
                 } else {
                     const TH hr = h3 - dt2h * (TH)rhs;
                     h2v = MH::max_(hr, TH(0.00));
-                    const u64 neg = vote(hr < 0) & sum;
+                    const u64 neg = vote(hr < 0) & A3;
                     if (neg) {
                         if (lanes(neg)) acc_clip += -(double)hr;
                     }
                 }
                 h2v = lanes(A3) ? h2v : TH(0.00);
-                if (lanes(sum)) {
-                    acc_vol += (double)h2v;
-                    if constexpr (kF32) acc_src += (double)(ql + rr * Pc - E);  // x dt2 below
-                    else acc_src += st.dt2 * ((double)ql + (double)rr * (double)Pc - (double)E);
+                acc_vol += (double)h2v;
+                if constexpr (kF32) {
+                    const T src = ql + rr * Pc - E;  // x dt2 below
+                    acc_src += (double)(lanes(A3) ? src : T(0));
+                } else {
+                    const double src = st.dt2 * ((double)ql + (double)rr * (double)Pc - (double)E);
+                    acc_src += lanes(A3) ? src : 0.0;
                 }
             }
         }
-        const unsigned row = put ? (unsigned)q * (unsigned)P : 0u;
-        h_out.store(outH, row, h2v, put);
-        um_out.store(outT, row, umpP, put);
-        vn_out.store(outT, row, vnpP, put);
+        // unconditional, for the count of accesses in flight; before the first
+        // row every lane's offset is kOutside
+        if (k == r0 + 3) {
+            row_out = (unsigned)r0 * (unsigned)P;
+            outT = colout ? (unsigned)j * (unsigned)sizeof(T) : kOutside;
+            outH = colout ? (unsigned)j * (unsigned)sizeof(TH) : kOutside;
+        }
+        h_out.store(outH, row_out, h2v);
+        um_out.store(outT, row_out, umpP);
+        vn_out.store(outT, row_out, vnpP);
+        row_out += k >= r0 + 3 ? (unsigned)P : 0u;
 
         // ---- rotate the row window ----
-        h3 = h2; h2 = h1; h1 = h0;
-        z2 = z1; z1 = z0;
-        A3 = A2; A2 = A1; A1 = A0;
-        W2 = W1; W1 = W0;
-        L2 = L1; L1 = L0;
-        u1 = u0; v1 = v0;
-        uu1_1 = uu1_0;
-        vv1_2 = vv1_1; vv1_1 = vv1_0;
-        px1 = px0; py1 = py0;
-        dzn1 = dzn0; dzw1 = dzw0;
-        nc2 = nc1; nc1 = nc0;
+        push(o);
         umnP = umn; vnnP = vnn;
         umpP = umpg; vnpP = vnpg;
-        FXQ = FXP; FXP = FX;
-        FYQ = FYP; FYP = FY;
         D1 = D0;
+        div1 = div0;
+        cut1 = cut;
     }
     // the outlet's discharge, where its cell is among this tile's outputs
     double acc_q = 0;
     if (orow >= r0 && orow < r1 && lanes(out_lane & out_cols)) acc_q = (double)qo_eff * s.dy;
 
     // ---- per-tile partial sums (fixed-order wave reductions) ----
+    if (!lanes(out_cols)) acc_vol = acc_src = acc_clip = 0;
     if constexpr (kF32) acc_src *= st.dt2;
     acc_vol = wave_sum(acc_vol);
     acc_src = wave_sum(acc_src);

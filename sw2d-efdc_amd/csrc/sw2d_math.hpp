@@ -113,14 +113,29 @@ static __constant__ const double kPowRecip[64] = {SW2D_POW_RECIP};
 static __constant__ const double kPowNlog[64] = {SW2D_POW_NLOG};
 static __constant__ const double kPowExp2[64] = {SW2D_POW_EXP2};
 
-// the tables where they lie, and a copy of them in LDS: recip, nlog, exp2 in a row
+// coefficients of pow1333_core: log1p from r^7 down to r^3, ln2 in two parts, the
+// exponent, 64 / ln2, ln2 / 64 in two parts, exp from r^6 down to r^3
+constexpr double kPowCoef[16] = {1.0 / 7.0, -1.0 / 6.0, 1.0 / 5.0, -0.25, 1.0 / 3.0, kLn2Hi, kLn2Lo, kManningExp,
+                                 64.0 * kInvLn2, kLn2Hi / 64.0, kLn2Lo / 64.0, 1.0 / 720.0, 1.0 / 120.0,
+                                 1.0 / 24.0, 1.0 / 6.0, 0.0};
+static __constant__ const double kPowCoefMem[16] = {
+    kPowCoef[0], kPowCoef[1], kPowCoef[2],  kPowCoef[3],  kPowCoef[4],  kPowCoef[5],  kPowCoef[6],  kPowCoef[7],
+    kPowCoef[8], kPowCoef[9], kPowCoef[10], kPowCoef[11], kPowCoef[12], kPowCoef[13], kPowCoef[14], kPowCoef[15]};
+
+// the tables where they lie, and a copy of them in LDS: recip, nlog, exp2 and the
+// coefficients in a row (LDS reads of 16 bytes in place of two moves a
+// coefficient; `zero` is 0, and keeps them from being held in registers)
 struct PowTables {
+    __device__ __forceinline__ double coef(int i) const { return kPowCoef[i]; }
     __device__ __forceinline__ double recip(int i) const { return kPowRecip[i]; }
     __device__ __forceinline__ double nlog(int i) const { return kPowNlog[i]; }
     __device__ __forceinline__ double exp2(int i) const { return kPowExp2[i]; }
 };
+constexpr int kPowLds = 192 + 16;
 struct PowTablesLds {
     const double *t;
+    int zero;
+    __device__ __forceinline__ double coef(int i) const { return t[192 + zero + i]; }
     __device__ __forceinline__ double recip(int i) const { return t[i]; }
     __device__ __forceinline__ double nlog(int i) const { return t[64 + i]; }
     __device__ __forceinline__ double exp2(int i) const { return t[128 + i]; }
@@ -135,24 +150,24 @@ __device__ __forceinline__ double pow1333_core(double x, const Tab &tab)
     const int i = (int)((b >> 46) & 63);
     const double m = __longlong_as_double((long long)((b & 0x000fffffffffffffULL) | 0x3ff0000000000000ULL));
     const double r = __builtin_fma(m, tab.recip(i), -1.0);
-    double q = 1.0 / 7.0;
-    q = __builtin_fma(r, q, -1.0 / 6.0);
-    q = __builtin_fma(r, q, 1.0 / 5.0);
-    q = __builtin_fma(r, q, -0.25);
-    q = __builtin_fma(r, q, 1.0 / 3.0);
+    double q = tab.coef(0);
+    q = __builtin_fma(r, q, tab.coef(1));
+    q = __builtin_fma(r, q, tab.coef(2));
+    q = __builtin_fma(r, q, tab.coef(3));
+    q = __builtin_fma(r, q, tab.coef(4));
     q = __builtin_fma(r, q, -0.5);
     const double lp = __builtin_fma(r * r, q, r);
     const double de = (double)e;
-    const double lx = __builtin_fma(de, kLn2Hi, __builtin_fma(de, kLn2Lo, tab.nlog(i) + lp));
-    const double t = kManningExp * lx;
-    const double kd = __builtin_rint(t * (64.0 * kInvLn2));
+    const double lx = __builtin_fma(de, tab.coef(5), __builtin_fma(de, tab.coef(6), tab.nlog(i) + lp));
+    const double t = tab.coef(7) * lx;
+    const double kd = __builtin_rint(t * tab.coef(8));
     const int k = (int)kd;
-    double rr = __builtin_fma(-kd, kLn2Hi / 64.0, t);
-    rr = __builtin_fma(-kd, kLn2Lo / 64.0, rr);
-    double p = 1.0 / 720.0;
-    p = __builtin_fma(rr, p, 1.0 / 120.0);
-    p = __builtin_fma(rr, p, 1.0 / 24.0);
-    p = __builtin_fma(rr, p, 1.0 / 6.0);
+    double rr = __builtin_fma(-kd, tab.coef(9), t);
+    rr = __builtin_fma(-kd, tab.coef(10), rr);
+    double p = tab.coef(11);
+    p = __builtin_fma(rr, p, tab.coef(12));
+    p = __builtin_fma(rr, p, tab.coef(13));
+    p = __builtin_fma(rr, p, tab.coef(14));
     p = __builtin_fma(rr, p, 0.5);
     const double P = __builtin_fma(rr * rr, p, rr);
     const double T = tab.exp2(k & 63);
