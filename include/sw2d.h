@@ -326,7 +326,7 @@ typedef struct sw2d_batch sw2d_batch;
 
 /* A batch on `device` owns one stream and a device memory pool of
  * pool_bytes; every member's arrays come from the pool.  All members share
- * `precision`.  tile_rows: rows per tile of members (0 = 32). */
+ * `precision`.  tile_rows: rows per tile of members (0 = automatic). */
 int sw2d_batch_create(int device, int precision, size_t pool_bytes, int tile_rows, sw2d_batch **out);
 /* Destroys the members still in the batch, then the batch. */
 int sw2d_batch_destroy(sw2d_batch *b);

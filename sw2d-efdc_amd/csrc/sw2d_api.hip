@@ -230,21 +230,30 @@ std::vector<int> round_fill_heights(long slots, const std::function<long(int)> &
 
 // Default tile height of the fused kernel (every tile is one wave): the height
 // whose launch the model of the row loop finds shortest.  A tile of H rows is a
-// chain of H + 4.5 row times (six halo rows, three of them without fluxes), and a
-// row takes r + w units with w waves on the SIMD: the chip works through whole
-// rounds of wave slots at full occupancy and the rest of the tiles at the
-// occupancy they reach.  r from launches of 2048^2, 556 x 701 and 331 x 1009
-// grids at heights of 2 to 80 rows; the model orders those as measured.
-int model_tile_rows(int prec, long slots, long simds, const std::function<long(int)> &blocks)
+// chain of H + 2.2 row times (the six halo rows; those without fluxes are short),
+// and a row takes r + w units with w waves on the SIMD.  A launch of one round of
+// wave slots takes a chain at the occupancy it reaches; a longer one works at full
+// occupancy, since slots are filled again as tiles end (at different times: a dry
+// tile is short), plus the end of its last tiles.  r and the last term from
+// launches of 2048^2, 1537 x 2311, 556 x 701, 331 x 1009 and 256^2 grids at heights
+// of 2 to 57 rows (2048^2 in FP32: 51.6 us at 15 rows, 56.5 at 12, 57.1 at 8).
+// FP32 and mixed launches that move more than the 256 MB cache holds are bound by
+// memory, which the last, long chains of tall tiles leave idle: 24 rows at most
+// there (4096^2 in FP32 142 us at 57 rows, 131 at 25, 137 at 10; 48 grids of
+// 128^2..1024^2 111.9 at 32, 108.1 at 20, 113.3 at 12).
+int model_tile_rows(int prec, long slots, long simds, long cells, const std::function<long(int)> &blocks)
 {
-    const double r = flux_bytes(prec) == 8 ? 2.1 : 3.3;
+    const bool f64 = flux_bytes(prec) == 8;
+    const double r = f64 ? 0.8 : 2.0, end = f64 ? 0.2 : 0.9;
     const double occ = (double)slots / simds;
+    const long bytes = cells * (2 * depth_bytes(prec) + 4 * flux_bytes(prec) + 8);
+    const int most = !f64 && bytes > (256L << 20) ? 24 : 80;
     int best = 2;
     double best_t = INFINITY;
-    for (int H = 2; H <= 80; H++) {
-        const long n = blocks(H), rest = n % slots;
-        const double w = (double)((rest + simds - 1) / simds);
-        const double t = (H + 4.5) * ((double)(n / slots) * (r + occ) + (rest ? r + w : 0.0));
+    for (int H = 2; H <= most; H++) {
+        const long n = blocks(H);
+        const double rounds = (double)n / slots;
+        const double t = (H + 2.2) * (n > slots ? rounds * (r + occ) + end : r + (double)((n + simds - 1) / simds));
         if (t < best_t) { best_t = t; best = H; }
     }
     return best;
@@ -256,7 +265,7 @@ int choose_tile_rows(const sw2d_handle *h)
     if (h->prm.tile_rows > 0) return std::min(h->prm.tile_rows, 512);
     const int feats = features_of(make_common(const_cast<sw2d_handle *>(h)));
     const long slots = wave_slots(h->device, h->prm.precision, feats);
-    return model_tile_rows(h->prm.precision, slots, 4L * device_cus(h->device),
+    return model_tile_rows(h->prm.precision, slots, 4L * device_cus(h->device), (long)h->R * h->C,
                            [&](int H) { return (long)blocks_at(h, H); });
 }
 

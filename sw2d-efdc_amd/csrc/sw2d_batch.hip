@@ -251,7 +251,7 @@ int sw2d_batch_create(int device, int precision, size_t pool_bytes, int tile_row
     b->graph_on = sw2d::graphs_enabled();
     b->device = device;
     b->precision = precision;
-    b->H = tile_rows > 0 ? tile_rows : 32;
+    b->H = tile_rows > 0 ? tile_rows : kBatchTileRows;
     auto bail = [&](hipError_t e, const char *what) {
         bhip(b, e, what);
         g_create_error = b->err;
@@ -307,7 +307,7 @@ size_t sw2d_batch_footprint(const sw2d_grid_desc *grid, const sw2d_params *param
     const size_t R = grid->rows, C = grid->cols;
     const size_t P = (size_t)round_up((int)C, 16);
     const size_t hb = depth_bytes(params->precision), fb = flux_bytes(params->precision);
-    const int H = params->tile_rows > 0 ? params->tile_rows : (tile_rows > 0 ? tile_rows : 32);
+    const int H = params->tile_rows > 0 ? params->tile_rows : (tile_rows > 0 ? tile_rows : kBatchTileRows);
     const size_t ntiles = ((C + 57) / 58) * ((R + H - 1) / H);
     size_t b = 0;
     b += 2 * pool_bytes_of(R * P * hb) + 4 * pool_bytes_of(R * P * fb);  // h, um, vn ping-pong

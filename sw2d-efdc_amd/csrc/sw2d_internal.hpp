@@ -163,6 +163,12 @@ struct Scenario {
 constexpr int kBookParts = 2;
 inline int book_blocks(int nbc) { return kBookParts + (nbc + 63) / 64; }
 
+// tile height of batch members that name none: between what
+// ensembles that fill the chip for several rounds and smaller ones want (a launch
+// of 24 grids of 128^2..1024^2 in FP64 takes 133 us at 20 rows, 147 at 32, 137 at
+// 12; 48 of them in FP32 108, 112, 113)
+constexpr int kBatchTileRows = 20;
+
 // one block of a batched launch: scenario and block within it
 struct TileRef {
     int sid, local;
