@@ -539,6 +539,7 @@ int sw2d_destroy(sw2d_handle *h)
     }
     if (h->stream) (void)hipStreamSynchronize(h->stream);
     snapshot_free(h);
+    readback_free(h);
     for (auto &ev : h->events) {
         (void)hipEventDestroy(ev.first);
         (void)hipEventDestroy(ev.second);
@@ -1034,13 +1035,18 @@ int sw2d_get_field(sw2d_handle *h, int field, double *out)
     const size_t RC = (size_t)h->R * h->C;
     HIPCHK(h, hipStreamSynchronize(h->stream));
     if (fused(h)) {
-        // derived fields go through an R*C FP64 buffer made on first use
-        int rc;
-        if (!h->scratch && (rc = dalloc(h, &h->scratch, RC))) return rc;
-        hipError_t e = launch_derive(h, field, h->scratch, 0, (long)RC);
-        if (e != hipSuccess) return hip_fail(h, e, "derive");
-        HIPCHK(h, hipMemcpyAsync(out, h->scratch, RC * 8, hipMemcpyDeviceToHost, h->stream));
-        HIPCHK(h, hipStreamSynchronize(h->stream));
+        if (readback_for(h)) {
+            hipError_t e = readback_field(h, field, out);
+            if (e != hipSuccess) return hip_fail(h, e, "derive");
+        } else {
+            // through an R*C FP64 buffer made on first use
+            int rc;
+            if (!h->scratch && (rc = dalloc(h, &h->scratch, RC))) return rc;
+            hipError_t e = launch_derive(h, field, h->scratch, 0, (long)RC);
+            if (e != hipSuccess) return hip_fail(h, e, "derive");
+            HIPCHK(h, hipMemcpyAsync(out, h->scratch, RC * 8, hipMemcpyDeviceToHost, h->stream));
+            HIPCHK(h, hipStreamSynchronize(h->stream));
+        }
         if (field == SW2D_FIELD_Z)
             for (size_t i = 0; i < RC; i++)
                 if (out[i] != out[i]) out[i] = h->grid.nodata;

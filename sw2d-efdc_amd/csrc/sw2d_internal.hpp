@@ -202,6 +202,7 @@ inline int features_of(const StepCommon &s)
 }
 
 struct SnapRing;   // asynchronous output copies (sw2d_output.hip)
+struct Readback;   // pinned buffers of sw2d_get_field (sw2d_output.hip)
 
 }  // namespace sw2d
 
@@ -277,6 +278,7 @@ struct sw2d_handle {
     long launches = 0;
     std::vector<void *> allocs;
     sw2d::SnapRing *snap = nullptr;     // sw2d_snapshot slots, made on first use
+    sw2d::Readback *readback = nullptr; // made on the first large sw2d_get_field
     std::string err;
 };
 

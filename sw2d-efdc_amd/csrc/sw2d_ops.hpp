@@ -132,6 +132,9 @@ int create_impl(const sw2d_grid_desc *grid, const double *z, const double *h0,
                 const HostImages *img = nullptr);
 // defined in sw2d_output.hip
 void snapshot_free(sw2d_handle *h);
+bool readback_for(sw2d_handle *h);
+hipError_t readback_field(sw2d_handle *h, int field, double *out);
+void readback_free(sw2d_handle *h);
 // defined in sw2d_batch.hip
 int batch_fit_tiles(sw2d_batch *b, int *tile_rows, int *retiled);
 
