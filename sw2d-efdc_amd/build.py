@@ -25,9 +25,12 @@ DRIVER = os.path.join(HERE, "sw2d-efdc")
 # forms gain nothing from it within the registers of five waves a SIMD.
 # Scheduling does not change what is rounded where.
 ILP_ITER = ["-mllvm", "-amdgpu-sched-strategy=iterative-ilp"]
-HIP_SOURCES = [("sw2d_api.hip", []), ("sw2d_fused64.hip", ILP_ITER),
-               ("sw2d_fused32.hip", ["-ffp-contract=on"]),
-               ("sw2d_fusedmix.hip", ["-ffp-contract=on"]), ("sw2d_plain.hip", []),
+# Its basic blocks that are jumped to start on 32 bytes, what one instruction
+# fetch brings: 331 x 1009 in FP32 15.9 -> 15.5 us, 48 grids 107.6 -> 106.5.
+ALIGN = ["-mllvm", "-align-all-nofallthru-blocks=5"]
+HIP_SOURCES = [("sw2d_api.hip", []), ("sw2d_fused64.hip", ILP_ITER + ALIGN),
+               ("sw2d_fused32.hip", ["-ffp-contract=on"] + ALIGN),
+               ("sw2d_fusedmix.hip", ["-ffp-contract=on"] + ALIGN), ("sw2d_plain.hip", []),
                ("sw2d_batch.hip", []), ("sw2d_server.hip", []), ("sw2d_output.hip", []),
                ("sw2d_host.cpp", [])]
 DRIVER_SOURCES = ["sw2d_driver.cpp", "sw2d_io.cpp", "sw2d_efdc_config.cpp", "sw2d_gefdc.cpp", "sw2d_lorp.cpp"]

@@ -11,16 +11,64 @@ struct StepTime {
     double t, dt, dt2, tm;
 };
 
+// Wave-wide reductions with a fixed combination order: lane i with lane i ^ 32,
+// then ^ 16 and so on (lane 0 holds the result; all lanes active).  The halves of
+// the wave and of its half rows are brought together by lane swaps, the rest by
+// DPP moves within rows of 16: after ^ 8 a row repeats itself, so a rotation by
+// 4 is ^ 4.  LDS permutes in their place wait for LDS six times a value.
+__device__ __forceinline__ int lane_hi(double v) { return (int)((unsigned long long)__double_as_longlong(v) >> 32); }
+__device__ __forceinline__ int lane_lo(double v) { return (int)__double_as_longlong(v); }
+__device__ __forceinline__ double lane_double(unsigned hi, unsigned lo)
+{
+    return __longlong_as_double((long long)((unsigned long long)hi << 32 | lo));
+}
+template <int CTRL> __device__ __forceinline__ double dpp_row(double v)
+{
+    return lane_double(__builtin_amdgcn_update_dpp(0, lane_hi(v), CTRL, 0xf, 0xf, true),
+                       __builtin_amdgcn_update_dpp(0, lane_lo(v), CTRL, 0xf, 0xf, true));
+}
+// f(own, other) over a row of 16 lanes whose values it combines
+template <typename Op> __device__ __forceinline__ double row_reduce(double v, const Op &f)
+{
+    v = f(v, dpp_row<0x128>(v));  // row_ror:8
+    v = f(v, dpp_row<0x124>(v));  // row_ror:4
+    v = f(v, dpp_row<0x4e>(v));   // quad_perm [2, 3, 0, 1]
+    return f(v, dpp_row<0xb1>(v));  // quad_perm [1, 0, 3, 2]
+}
+template <typename Op> __device__ __forceinline__ double wave_reduce(double v, const Op &f)
+{
+    {
+        const auto h = __builtin_amdgcn_permlane32_swap(lane_hi(v), lane_hi(v), false, false);
+        const auto l = __builtin_amdgcn_permlane32_swap(lane_lo(v), lane_lo(v), false, false);
+        v = f(lane_double(h[0], l[0]), lane_double(h[1], l[1]));
+    }
+    {
+        const auto h = __builtin_amdgcn_permlane16_swap(lane_hi(v), lane_hi(v), false, false);
+        const auto l = __builtin_amdgcn_permlane16_swap(lane_lo(v), lane_lo(v), false, false);
+        v = f(lane_double(h[0], l[0]), lane_double(h[1], l[1]));
+    }
+    return row_reduce(v, f);
+}
+__device__ __forceinline__ double wave_sum(double v)
+{
+    return wave_reduce(v, [](double a, double b) { return a + b; });
+}
+__device__ __forceinline__ double wave_max(double v)
+{
+    return wave_reduce(v, [](double a, double b) { return (b > a) ? b : a; });
+}
+__device__ __forceinline__ double wave_min(double v)
+{
+    return wave_reduce(v, [](double a, double b) { return (b < a) ? b : a; });
+}
+
 // the CFL minimum of a clock slot: one partial minimum a lane, combined over
 // the wave (all lanes active; the result is the same in every lane)
 __device__ __forceinline__ double clock_cfl(const Clock &ck)
 {
-    static_assert((kCflSlots & (kCflSlots - 1)) == 0 && kCflSlots <= 64, "");
-    double m = __longlong_as_double((long long)ck.cfl[threadIdx.x & (kCflSlots - 1)].bits);
-    for (int off = kCflSlots / 2; off >= 1; off >>= 1) {
-        const double o = __shfl_xor(m, off, 64);
-        m = (o < m) ? o : m;
-    }
+    static_assert(kCflSlots == 16, "a row of lanes");
+    const double m = row_reduce(__longlong_as_double((long long)ck.cfl[threadIdx.x & (kCflSlots - 1)].bits),
+                                [](double a, double b) { return (b < a) ? b : a; });
     const long long b = __double_as_longlong(m);  // uniform: into scalar registers
     const unsigned lo = __builtin_amdgcn_readfirstlane((int)b), hi = __builtin_amdgcn_readfirstlane((int)(b >> 32));
     return __longlong_as_double((long long)((unsigned long long)hi << 32 | lo));
@@ -96,29 +144,6 @@ __device__ __forceinline__ double storm_factor(double d, double sigma)
 __device__ __forceinline__ bool storm_live(const StepCommon &s, double t)
 {
     return s.storm_on && (t >= s.st_t0) && (t < s.st_t1);
-}
-
-// wave-wide reductions with a fixed combination order (lane 0 holds the result)
-__device__ __forceinline__ double wave_sum(double v)
-{
-    for (int off = 32; off >= 1; off >>= 1) v += __shfl_xor(v, off, 64);
-    return v;
-}
-__device__ __forceinline__ double wave_max(double v)
-{
-    for (int off = 32; off >= 1; off >>= 1) {
-        double o = __shfl_xor(v, off, 64);
-        v = (o > v) ? o : v;
-    }
-    return v;
-}
-__device__ __forceinline__ double wave_min(double v)
-{
-    for (int off = 32; off >= 1; off >>= 1) {
-        double o = __shfl_xor(v, off, 64);
-        v = (o < v) ? o : v;
-    }
-    return v;
 }
 
 // inflow rate of one coupling record (couple_BC_efdc, SW2D-EFDC.cu:764-821)

@@ -76,6 +76,9 @@ __device__ __forceinline__ unsigned any_lane(u64 m)
     asm("s_bcnt1_i32_b64 %0, %1" : "=s"(n) : "s"(m) : "scc");
     return n < 1u ? n : 1u;
 }
+// keeps a rarely taken branch one: the compiler would make selects of it, which
+// every row would execute
+__device__ __forceinline__ void keep_branch() { asm volatile(""); }
 // a wave-uniform condition that the compiler cannot see to be uniform
 __device__ __forceinline__ bool uniform(bool p) { return __builtin_amdgcn_readfirstlane((int)p) != 0; }
 
@@ -642,6 +645,7 @@ fused_step(const Scenario *__restrict__ scen, const TileRef *__restrict__ tiles,
         if ((flow & 13u) || g == orow) {
             T Pc = P_land, E = T(0.000);
             if (!even) {
+                keep_branch();
                 const bool wet = h2 > ewl;
                 Pc = wet ? P_lake : P_land;
                 E = wet ? ev1t : T(0.000);
@@ -685,13 +689,14 @@ fused_step(const Scenario *__restrict__ scen, const TileRef *__restrict__ tiles,
         // ---- second continuity of row q = k-3 at time t + dt; store ----
         const int q = k - 3;
         TH h2v = 0;
+        T src = 0;
         if (k >= r0 + 3) {
             if (calm2 && !(flow & 52u) && q != orow && !vote(!(h3 >= TH(0)))) {
                 h2v = lanes(A3) ? h3 : TH(0);
-                acc_vol += (double)h2v;
             } else {
                 T Pc = P_land, E = T(0.000);
                 if (!even) {
+                    keep_branch();
                     const bool wet = h3 > ewl;
                     Pc = wet ? P_lake : P_land;
                     E = wet ? ev2t : T(0.000);
@@ -760,19 +765,17 @@ fused_step(const Scenario *__restrict__ scen, const TileRef *__restrict__ tiles,
                     }
                 }
                 h2v = lanes(A3) ? h2v : TH(0.00);
-                acc_vol += (double)h2v;
-                if constexpr (kF32) {
-                    const T src = ql + rr * Pc - E;  // x dt2 below
-                    acc_src += (double)(lanes(A3) ? src : T(0));
-                } else {
-                    const double src = st.dt2 * ((double)ql + (double)rr * (double)Pc - (double)E);
-                    acc_src += lanes(A3) ? src : 0.0;
-                }
+                if constexpr (kF32) src = ql + rr * Pc - E;  // x dt2 below
+                else src = st.dt2 * ((double)ql + (double)rr * (double)Pc - (double)E);
+                src = lanes(A3) ? src : T(0);
             }
         }
+        acc_vol += (double)h2v;
+        acc_src += (double)src;
         // unconditional, for the count of accesses in flight; before the first
         // row every lane's offset is kOutside
         if (k == r0 + 3) {
+            keep_branch();
             row_out = (unsigned)r0 * (unsigned)P;
             outT = colout ? (unsigned)j * (unsigned)sizeof(T) : kOutside;
             outH = colout ? (unsigned)j * (unsigned)sizeof(TH) : kOutside;
