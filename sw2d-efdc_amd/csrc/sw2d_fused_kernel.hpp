@@ -79,9 +79,6 @@ __device__ __forceinline__ unsigned any_lane(u64 m)
 // keeps a rarely taken branch one: the compiler would make selects of it, which
 // every row would execute
 __device__ __forceinline__ void keep_branch() { asm volatile(""); }
-// a wave-uniform condition that the compiler cannot see to be uniform
-__device__ __forceinline__ bool uniform(bool p) { return __builtin_amdgcn_readfirstlane((int)p) != 0; }
-
 // One scenario array, read and written through a buffer resource (base and
 // range in scalar registers): a lane's byte offset within the row stays in one
 // register for the whole tile and the row's byte offset is scalar, so a row
@@ -315,8 +312,10 @@ fused_step(const Scenario *__restrict__ scen, const TileRef *__restrict__ tiles,
     const Arr<const double> zg(kH32 ? d.dz : d.z, cells);
     const bool map_on = kMap && s.ncls_on;
     const Arr<uint8_t> cls_in(map_on ? (const void *)d.cls : (const void *)d.z, map_on ? cells : 0u);
-    __shared__ T nt_s[kMaxClasses];  // Manning coefficients of the classes
-    if (kMap && lane < kMaxClasses) nt_s[lane] = (T)s.ntab[lane];
+    // Manning coefficients of the classes; without a map every cell reads class
+    // 0 (an empty array), which is the scenario's coefficient
+    __shared__ T nt_s[kMaxClasses];
+    if (kMap && lane < kMaxClasses) nt_s[lane] = (T)(map_on ? s.ntab[lane] : s.rn);
     // FP64: the tables of the power in LDS.  Reads of them from memory share the
     // counter of the row loads, and waiting for one of the former waits for the
     // next row as well: four such waits a row with friction on both faces.  24
@@ -424,9 +423,15 @@ fused_step(const Scenario *__restrict__ scen, const TileRef *__restrict__ tiles,
     const TH ewl = (TH)s.EV_WL_min;
     // no water is added or taken in the second continuity: a row without
     // fluxes then keeps its depths
-    const bool calm2 = uniform(!storm_on && nst == 0 && rr2 == 0.0 && ev2 == 0.0);
+    const bool calm2 = !storm_on && nst == 0 && rr2 == 0.0 && ev2 == 0.0;
     // one forcing for all depths (no evaporation, the same fraction of the rain)
-    const bool even = uniform(s.P_lake == s.P_land && ev1 == 0.0 && ev2 == 0.0);
+    const bool even = s.P_lake == s.P_land && ev1 == 0.0 && ev2 == 0.0;
+    // the scenario's conditions as bits of one register, tested where they are
+    // needed (as conditions they take two registers each, too many to keep)
+    enum : unsigned { kOnStorm = 1, kOnStorm1 = 2, kOnStorm2 = 4, kOnCalm = 8, kOnEven = 16 };
+    const unsigned on_bits = (unsigned)__builtin_amdgcn_readfirstlane(
+        (storm_on ? kOnStorm : 0u) | (storm1 ? kOnStorm1 : 0u) | (storm2 ? kOnStorm2 : 0u) |
+        (calm2 ? kOnCalm : 0u) | (even ? kOnEven : 0u));
     const int out_edge = __builtin_amdgcn_readfirstlane(s.out_edge);
 
     // the outlet's row, where its column is among this wave's lanes, and its lane
@@ -485,7 +490,7 @@ fused_step(const Scenario *__restrict__ scen, const TileRef *__restrict__ tiles,
         o.W = vote(o.h > thh);
         o.L = vote(o.h < thh);
         o.nc = rn;
-        if constexpr (kMap) o.nc = map_on ? nt_s[cl] : rn;
+        if constexpr (kMap) o.nc = nt_s[cl];
 
         // ---- face depths and velocities (hm_hn, uu1_vv1) ----
         // (row 0's north and column 0's west faces carry no flux, so their
@@ -533,6 +538,8 @@ fused_step(const Scenario *__restrict__ scen, const TileRef *__restrict__ tiles,
     // be a wait for the stores of the row before in every later row)
     __builtin_amdgcn_s_waitcnt(0x0070);
     for (int k = r0; k < kend; ++k) {
+        unsigned on = on_bits;
+        asm volatile("" : "+s"(on));
         const Front o = front(k);
         const TH hm0d = o.hm, hn0d = o.hn;
         const T hm0 = (T)hm0d, hn0 = (T)hn0d, uu1_0 = o.uu1, vv1_0 = o.vv1, px0 = o.px, py0 = o.py;
@@ -644,17 +651,17 @@ fused_step(const Scenario *__restrict__ scen, const TileRef *__restrict__ tiles,
         unsigned cut = 0;  // fluxes of row g taken out: bit 0 north faces, bit 1 west faces
         if ((flow & 13u) || g == orow) {
             T Pc = P_land, E = T(0.000);
-            if (!even) {
+            if (!(on & kOnEven)) {
                 keep_branch();
                 const bool wet = h2 > ewl;
                 Pc = wet ? P_lake : P_land;
                 E = wet ? ev1t : T(0.000);
             }
             T rr = rr1t;
-            if (storm_on) {
+            if (kStorm && (on & kOnStorm)) {
                 const T gy = gy_s[0][g - (r0 - 5)];
                 if constexpr (kF32) rr = pk1 * gy;
-                else rr = storm1 ? (T)(s.st_peak * (gx1 * gy)) : T(0);
+                else rr = (on & kOnStorm1) ? (T)(s.st_peak * (gx1 * gy)) : T(0);
             }
             T ql = 0;
             for (int i = 0; i < nst; ++i)
@@ -691,21 +698,21 @@ fused_step(const Scenario *__restrict__ scen, const TileRef *__restrict__ tiles,
         TH h2v = 0;
         T src = 0;
         if (k >= r0 + 3) {
-            if (calm2 && !(flow & 52u) && q != orow && !vote(!(h3 >= TH(0)))) {
+            if ((on & kOnCalm) && !(flow & 52u) && q != orow && !vote(!(h3 >= TH(0)))) {
                 h2v = lanes(A3) ? h3 : TH(0);
             } else {
                 T Pc = P_land, E = T(0.000);
-                if (!even) {
+                if (!(on & kOnEven)) {
                     keep_branch();
                     const bool wet = h3 > ewl;
                     Pc = wet ? P_lake : P_land;
                     E = wet ? ev2t : T(0.000);
                 }
                 T rr = rr2t;
-                if (storm_on) {
+                if (kStorm && (on & kOnStorm)) {
                     const T gy = gy_s[1][q - (r0 - 6)];
                     if constexpr (kF32) rr = pk2 * gy;
-                    else rr = storm2 ? (T)(s.st_peak * (gx2 * gy)) : T(0);
+                    else rr = (on & kOnStorm2) ? (T)(s.st_peak * (gx2 * gy)) : T(0);
                 }
                 T ql = 0;
                 for (int i = 0; i < nst; ++i)
