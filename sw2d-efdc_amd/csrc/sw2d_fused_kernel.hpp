@@ -461,10 +461,13 @@ fused_step(const Scenario *__restrict__ scen, const TileRef *__restrict__ tiles,
     unsigned cut1 = 0;
 
     // sums over all lanes; those outside the output columns are dropped at the end
-    double acc_vol = 0, acc_src = 0, acc_clip = 0;
-    // CFL: the largest |u| + sqrt(g h) per direction; min_f dx / s_f = dx / max_f s_f
-    // because rounding dx / s is monotone in s
-    T smax_x = 0, smax_y = 0;
+    // (the clipped volume, which few rows add to, in LDS)
+    double acc_vol = 0, acc_src = 0;
+    __shared__ double clip_s[64];
+    clip_s[lane] = 0.0;
+    // CFL: the largest |u| + sqrt(g h) of either direction; min_f dx / s_f =
+    // dx / max_f s_f because rounding dx / s is monotone in s (and dy = dx)
+    T smax = 0;
 
     // row k: what the rows after it need of it
     struct Front {
@@ -550,11 +553,11 @@ fused_step(const Scenario *__restrict__ scen, const TileRef *__restrict__ tiles,
             // CFL candidates of the incoming state on the faces of row k
             if (lanes(A0 & A1 & out_cols & vote(hm0d > thh))) {
                 const T w = M::abs_(uu1_0) + M::sqrt_(gg * hm0);
-                smax_x = (w > smax_x) ? w : smax_x;
+                smax = (w > smax) ? w : smax;
             }
             if (lanes(A0 & (A0 << 1) & out_cols & vote(hn0d > thh))) {
                 const T w = M::abs_(vv1_0) + M::sqrt_(gg * hn0);
-                smax_y = (w > smax_y) ? w : smax_y;
+                smax = (w > smax) ? w : smax;
             }
         }
 
@@ -760,7 +763,7 @@ fused_step(const Scenario *__restrict__ scen, const TileRef *__restrict__ tiles,
                     // (exact: 48 bits suffice) is needed only then
                     const u64 neg = vote(sm <= T(0)) & (vote(sm < T(0)) | vote(er < T(0)));
                     if (neg) {
-                        if (lanes(neg & A3)) acc_clip += -((double)sm + (double)er);
+                        if (lanes(neg & A3)) clip_s[lane] += -((double)sm + (double)er);
                         h2v = lanes(neg) ? TH(0) : h2v;
                     }
                 } else {
@@ -768,7 +771,7 @@ fused_step(const Scenario *__restrict__ scen, const TileRef *__restrict__ tiles,
                     h2v = MH::max_(hr, TH(0.00));
                     const u64 neg = vote(hr < 0) & A3;
                     if (neg) {
-                        if (lanes(neg)) acc_clip += -(double)hr;
+                        if (lanes(neg)) clip_s[lane] += -(double)hr;
                     }
                 }
                 h2v = lanes(A3) ? h2v : TH(0.00);
@@ -805,6 +808,7 @@ fused_step(const Scenario *__restrict__ scen, const TileRef *__restrict__ tiles,
     if (orow >= r0 && orow < r1 && lanes(out_lane & out_cols)) acc_q = (double)qo_eff * s.dy;
 
     // ---- per-tile partial sums (fixed-order wave reductions) ----
+    double acc_clip = clip_s[lane];
     if (!lanes(out_cols)) acc_vol = acc_src = acc_clip = 0;
     if constexpr (kF32) acc_src *= st.dt2;
     acc_vol = wave_sum(acc_vol);
@@ -813,10 +817,8 @@ fused_step(const Scenario *__restrict__ scen, const TileRef *__restrict__ tiles,
     acc_q = wave_sum(acc_q);
     double cfl = INFINITY;
     if (adapt) {
-        const double mx = wave_max((double)smax_x), my = wave_max((double)smax_y);
-        const double wx = mx > 0.0 ? s.dx / mx : INFINITY;
-        const double wy = my > 0.0 ? s.dy / my : INFINITY;
-        cfl = (wx < wy) ? wx : wy;
+        const double m = wave_max((double)smax);
+        cfl = m > 0.0 ? s.dx / m : INFINITY;
     }
     if (lane == 0) {
         Partial p;
