@@ -192,15 +192,14 @@ __device__ __forceinline__ PowTablesLds pow_tables(const double *t)
 constexpr int kMaxTileRows = 512;
 
 // Waves per SIMD that the registers have to leave room for.  Each of them issues
-// about one instruction in 5.5 cycles, so SIMDs are filled by more of them: a
-// row takes a wave (3.3 + w) units of time beside w - 1 others in the FP32 and
-// mixed forms, (2.1 + w) in FP64 (2048^2 and 331 x 1009 grids at w = 1 to 5).
-// 3 against 2 in FP64: 2048^2 134 -> 125 us, 24 grids of 128^2..1024^2 the same;
-// 5 against 4 in FP32: 2048^2 59.0 -> 56.8.  Six waves (80 registers) spill, and
-// so does the instantiation with every feature at these counts: 556 x 701 in
-// FP64, two waves a SIMD whatever its registers, 27.0 us without, 29.5 with.
+// about one instruction in 4 to 5 cycles, so SIMDs are filled by more of them: a
+// row takes a wave (2.0 + w) units of time beside w - 1 others in the FP32 and
+// mixed forms, (0.8 + w) in FP64 (2048^2 and 331 x 1009 grids at w = 1 to 5).
+// 3 against 2 in FP64: 2048^2 134 -> 125 us when it came; 4 (128 registers) spill:
+// 107 -> 137.  5 against 4 in FP32: 2048^2 59.0 -> 56.8 when it came; 6 (80
+// registers) spill in the storm's instantiation: 50.4 -> 53.1.
 template <typename T, int F>
-constexpr int kMinWaves = (sizeof(T) == 8 ? 3 : 5) - ((F & kFeatSources) ? 1 : 0);
+constexpr int kMinWaves = (sizeof(T) == 8 ? 3 : 5);
 
 // F: the features (kFeat*) this instantiation handles.  A feature missing
 // from F is compiled out (its uniforms, branches and loops), which the host
