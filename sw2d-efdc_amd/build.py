@@ -29,8 +29,8 @@ ILP_ITER = ["-mllvm", "-amdgpu-sched-strategy=iterative-ilp"]
 # fetch brings: 331 x 1009 in FP32 15.9 -> 15.5 us, 48 grids 107.6 -> 106.5.
 ALIGN = ["-mllvm", "-align-all-nofallthru-blocks=5"]
 HIP_SOURCES = [("sw2d_api.hip", []), ("sw2d_fused64.hip", ILP_ITER + ALIGN),
-               ("sw2d_fused32.hip", ["-ffp-contract=on"] + ALIGN),
-               ("sw2d_fusedmix.hip", ["-ffp-contract=on"] + ALIGN), ("sw2d_plain.hip", []),
+               ("sw2d_fused32.hip", ["-ffp-contract=on"] + ILP_ITER + ALIGN),
+               ("sw2d_fusedmix.hip", ["-ffp-contract=on"] + ILP_ITER + ALIGN), ("sw2d_plain.hip", []),
                ("sw2d_batch.hip", []), ("sw2d_server.hip", []), ("sw2d_output.hip", []),
                ("sw2d_host.cpp", [])]
 DRIVER_SOURCES = ["sw2d_driver.cpp", "sw2d_io.cpp", "sw2d_efdc_config.cpp", "sw2d_gefdc.cpp", "sw2d_lorp.cpp"]
