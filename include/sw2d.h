@@ -222,7 +222,9 @@ int sw2d_time(sw2d_handle *h, double *time, long *mstep, double *dt2_next);
 /* Copy one field (rows*cols doubles) to caller memory; derived fields are
  * computed from the current state as hm_hn/uu1_vv1/uu_vv/uua_vva do
  * (362-522).  Replaces the D2H copies at output times (4900, 4976, 5026,
- * 5042, 5058).  Synchronises. */
+ * 5042, 5058).  Synchronises.  The first call on a stand-alone fused handle
+ * allocates a buffer that stays with it: R*C doubles on the device, or 8 MiB of
+ * pinned host memory for grids of 2^20 cells or more. */
 int sw2d_get_field(sw2d_handle *h, int field, double *out);
 
 /* sw2d_get_field without any device allocation.  No counterpart in the
@@ -231,7 +233,7 @@ int sw2d_get_field(sw2d_handle *h, int field, double *out);
  * hipMalloc).  The same values as sw2d_get_field, but a derived field of a
  * fused handle is staged through a fixed 16 MiB device array that each GPU
  * holds from the library's load until the process ends, in chunks of whole
- * rows, instead of the R*C buffer sw2d_get_field allocates on first use.
+ * rows, instead of the buffer sw2d_get_field allocates on first use.
  * Grids with more than 2^21 columns are refused (SW2D_E_ARG).  Calls on one
  * GPU share its array: the library serialises them within a process (a call
  * holds the array until its copy has finished), so calls that overlap on one

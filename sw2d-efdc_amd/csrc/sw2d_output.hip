@@ -13,7 +13,7 @@
 #include <condition_variable>
 #include <memory>
 #include <mutex>
-#include <system_error>
+#include <exception>
 #include <thread>
 
 #include "sw2d_ops.hpp"
@@ -68,7 +68,7 @@ void snapshot_free(sw2d_handle *h)
 // into pinned buffers (no device copy of the field), and two threads with two
 // buffers each move them on: 46.9 GB/s with chunks of 2 MiB (1 thread 29.0, 4
 // threads 48.0; chunks of 1 MiB 41.7; DMA into the pinned buffers 40.0).  The
-// three fields of a 4096^2 grid 24.7 -> 10 ms, of 2048^2 6.9 -> 3.  Making the
+// three fields of a 4096^2 grid 24.7 -> 10.5 ms, of 2048^2 6.9 -> 3.3.  Making the
 // buffers takes about 1 ms, so fields below kReadbackMin go the plain way.
 // ---------------------------------------------------------------------------
 constexpr size_t kReadbackMin = 1u << 20;                // values of a field: 8 MiB
@@ -145,7 +145,7 @@ hipError_t readback_field(sw2d_handle *h, int field, double *out)
             err[1] = hipSetDevice(h->device);
             if (err[1] == hipSuccess) lane(1, 2);
         });
-    } catch (const std::system_error &) {
+    } catch (const std::exception &) {
         // no thread to be had: one lane
     }
     if (second.joinable()) {
