@@ -455,7 +455,8 @@ typedef struct sw2d_server_stats {
 /* tile_rows: tile height of every request that names none (0 = adaptive:
  * after each admission or retirement the running requests are retiled to the
  * height that fills whole rounds of wave slots, the fewest rounds with a
- * height of at most 80, else 32; results are those of any fixed height, the
+ * height of at most 80, else 32, or where their launch is bound by memory to
+ * the one a model of the kernel finds shortest; results are those of any fixed height, the
  * volume ledger to rounding).
  * slice_iters: iterations per batch step between admissions (0 = 60).
  * The server's batch interleaves the running requests' tiles block by block

@@ -241,13 +241,17 @@ std::vector<int> round_fill_heights(long slots, const std::function<long(int)> &
 // memory, which the last, long chains of tall tiles leave idle: 24 rows at most
 // there (4096^2 in FP32 142 us at 57 rows, 131 at 25, 137 at 10; 48 grids of
 // 128^2..1024^2 111.9 at 32, 108.1 at 20, 113.3 at 12).
+bool memory_bound(int prec, long cells)
+{
+    const long bytes = cells * (2 * depth_bytes(prec) + 4 * flux_bytes(prec) + 8);
+    return flux_bytes(prec) == 4 && bytes > (256L << 20);
+}
 int model_tile_rows(int prec, long slots, long simds, long cells, const std::function<long(int)> &blocks)
 {
     const bool f64 = flux_bytes(prec) == 8;
     const double r = f64 ? 0.8 : 2.0, end = f64 ? 0.2 : 0.9;
     const double occ = (double)slots / simds;
-    const long bytes = cells * (2 * depth_bytes(prec) + 4 * flux_bytes(prec) + 8);
-    const int most = !f64 && bytes > (256L << 20) ? 24 : 80;
+    const int most = memory_bound(prec, cells) ? 24 : 80;
     int best = 2;
     double best_t = INFINITY;
     for (int H = 2; H <= most; H++) {

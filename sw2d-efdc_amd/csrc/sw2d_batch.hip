@@ -189,11 +189,11 @@ size_t pool_bytes_of(size_t bytes) { return Pool::rounded(bytes); }
 
 namespace sw2d {
 
-// Round-filling tile height for the members still running (a member with a
-// height of its own keeps it): the fewest whole rounds of wave slots whose
-// height is at most 80, else 32 when even six rounds need taller tiles (on
-// the serving mix two rounds at H ~ 55 beat three at H ~ 37 by 1%: fewer halo
-// rows per output row).  The
+// Tile height for the members still running (a member with a height of its own
+// keeps it).  Launches that memory bounds take the height of the model of the row
+// loop: the served mix with 64 Mi running cells 1.10e11 cell-updates/s at
+// round-filling heights, 1.23e11 at the model's.  Others fill whole rounds of wave
+// slots, the fewest whose height is at most 80, else 32.  The
 // running members are retiled to it and new members start at it.  A member
 // whose retile finds no pool memory keeps its height (members of one launch
 // may differ in height).  *retiled counts the members moved.
@@ -212,14 +212,21 @@ int batch_fit_tiles(sw2d_batch *b, int *tile_rows, int *retiled)
     }
     if (!run.empty()) {
         const long slots = wave_slots(b->device, b->precision, feats);
-        const std::vector<int> fit = round_fill_heights(slots, [&](int H) {
+        long cells = 0;
+        for (const sw2d_handle *h : run) cells += (long)h->R * h->C;
+        auto blocks = [&](int H) {
             long n = 0;
             for (const sw2d_handle *h : run) n += blocks_at(h, h->prm.tile_rows > 0 ? h->prm.tile_rows : H);
             return n;
-        });
+        };
         int best = 32;
-        for (auto it = fit.rbegin(); it != fit.rend(); ++it)
-            if (*it <= 80) { best = *it; break; }
+        if (memory_bound(b->precision, cells)) {
+            best = model_tile_rows(b->precision, slots, 4L * device_cus(b->device), cells, blocks);
+        } else {
+            const std::vector<int> fit = round_fill_heights(slots, blocks);
+            for (auto it = fit.rbegin(); it != fit.rend(); ++it)
+                if (*it <= 80) { best = *it; break; }
+        }
         b->H = best;
         for (sw2d_handle *h : run) {
             if (h->prm.tile_rows > 0 || h->H == best) continue;

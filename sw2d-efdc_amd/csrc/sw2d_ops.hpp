@@ -105,6 +105,7 @@ int fused_blocks(const sw2d_handle *h);
 Scenario make_scenario(sw2d_handle *h);
 int choose_tile_rows(const sw2d_handle *h);
 int device_cus(int device);
+bool memory_bound(int prec, long cells);
 int model_tile_rows(int prec, long slots, long simds, long cells, const std::function<long(int)> &blocks);
 long wave_slots(int device, int prec, int features);
 int blocks_at(const sw2d_handle *h, int H);
