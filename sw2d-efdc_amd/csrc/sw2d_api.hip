@@ -90,7 +90,7 @@ int upload_desc(sw2d_handle *h)
     if (!h->desc_dirty) return SW2D_OK;
     const Scenario d = make_scenario(h);
     HIPCHK(h, hipMemcpyAsync(h->dscen, &d, sizeof d, hipMemcpyHostToDevice, h->stream));
-    HIPCHK(h, launch_forcing(h->stream, h->dscen, 1));
+    HIPCHK(h, launch_forcing(h->prm.precision, h->stream, h->dscen, 1));
     HIPCHK(h, hipStreamSynchronize(h->stream));
     h->desc_dirty = false;
     return SW2D_OK;

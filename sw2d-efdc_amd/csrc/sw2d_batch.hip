@@ -119,7 +119,7 @@ int rebuild(sw2d_batch *b)
     }
     if (top > 0) {
         BCHK(b, hipMemcpy(b->dscen, desc.data(), sizeof(Scenario) * top, hipMemcpyHostToDevice));
-        BCHK(b, launch_forcing(b->stream, b->dscen, top));
+        BCHK(b, launch_forcing(b->precision, b->stream, b->dscen, top));
     }
     if (!tiles.empty())
         BCHK(b, hipMemcpy(b->dtiles, tiles.data(), sizeof(TileRef) * tiles.size(), hipMemcpyHostToDevice));

@@ -39,6 +39,10 @@ hipError_t launch_fused_f32(hipStream_t stream, const Scenario *scen, const Tile
 {
     return launch_fused_impl<float, float>(stream, scen, tiles, nblocks, phase, features, lds);
 }
+hipError_t launch_forcing_f32(hipStream_t stream, const Scenario *scen, int n)
+{
+    return launch_forcing_impl<float, float>(stream, scen, n);
+}
 int fused_waves_per_cu_f32(int features) { return fused_waves_per_cu_impl<float, float>(features); }
 hipError_t launch_init_f32(sw2d_handle *h) { return launch_init_impl<float, float>(h); }
 hipError_t launch_bed_steps(sw2d_handle *h)

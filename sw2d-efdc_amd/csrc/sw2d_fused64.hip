@@ -15,6 +15,10 @@ hipError_t launch_fused_f64(hipStream_t stream, const Scenario *scen, const Tile
 {
     return launch_fused_impl<double, double>(stream, scen, tiles, nblocks, phase, features, lds);
 }
+hipError_t launch_forcing_f64(hipStream_t stream, const Scenario *scen, int n)
+{
+    return launch_forcing_impl<double, double>(stream, scen, n);
+}
 int fused_waves_per_cu_f64(int features) { return fused_waves_per_cu_impl<double, double>(features); }
 hipError_t launch_init_f64(sw2d_handle *h) { return launch_init_impl<double, double>(h); }
 hipError_t launch_derive_f64(sw2d_handle *h, int field, double *out, long first, long count)
@@ -25,19 +29,6 @@ hipError_t launch_derive_f64(sw2d_handle *h, int field, double *out, long first,
 hipError_t launch_peek(sw2d_handle *h, const StepCommon &sc)
 {
     hipLaunchKernelGGL(peek_kernel, dim3(1), dim3(64), 0, h->stream, sc, h->peek);
-    return hipGetLastError();
-}
-
-// one wave a descriptor; a slot without a member is all zeros
-__global__ void __launch_bounds__(64) forcing_kernel(const Scenario *scen)
-{
-    const StepCommon &s = scen[blockIdx.x].s;
-    if (s.clk) note_forcing(s, s.slot_a, s.clk[s.slot_a].t, threadIdx.x);
-}
-
-hipError_t launch_forcing(hipStream_t stream, const Scenario *scen, int n)
-{
-    hipLaunchKernelGGL(forcing_kernel, dim3(n), dim3(64), 0, stream, scen);
     return hipGetLastError();
 }
 

@@ -828,6 +828,24 @@ fused_step(const Scenario *__restrict__ scen, const TileRef *__restrict__ tiles,
     }
 }
 
+// The forcing of every descriptor's current iteration, one wave a descriptor; a
+// slot without a member is all zeros.  In each form's own unit: the units fuse
+// multiply-adds under different rules, and a rate has to round the same here and
+// where fused_step evaluates it for the next iteration.
+template <typename T, typename TH>
+__global__ void __launch_bounds__(64) forcing_kernel(const Scenario *scen)
+{
+    const StepCommon &s = scen[blockIdx.x].s;
+    if (s.clk) note_forcing(s, s.slot_a, s.clk[s.slot_a].t, threadIdx.x);
+}
+
+template <typename T, typename TH>
+static hipError_t launch_forcing_impl(hipStream_t stream, const Scenario *scen, int n)
+{
+    hipLaunchKernelGGL((forcing_kernel<T, TH>), dim3(n), dim3(64), 0, stream, scen);
+    return hipGetLastError();
+}
+
 // initial CFL minimum of the state (adaptive mode)
 template <typename T, typename TH>
 __global__ void __launch_bounds__(256) init_cfl(const TH *h, const T *um, const T *vn,

@@ -347,7 +347,9 @@ hipError_t launch_derive_mix(sw2d_handle *h, int field, double *out_dev, long fi
 hipError_t launch_peek(sw2d_handle *h, const StepCommon &sc);
 // the forcing of each descriptor's current iteration (clock slot s.slot_a)
 // into its clock, after the descriptors changed
-hipError_t launch_forcing(hipStream_t stream, const Scenario *scen, int n);
+hipError_t launch_forcing_f64(hipStream_t stream, const Scenario *scen, int n);
+hipError_t launch_forcing_f32(hipStream_t stream, const Scenario *scen, int n);
+hipError_t launch_forcing_mix(hipStream_t stream, const Scenario *scen, int n);
 int fused_waves_per_cu_f64(int features);  // resident one-wave blocks per CU
 int fused_waves_per_cu_f32(int features);
 int fused_waves_per_cu_mix(int features);
@@ -367,6 +369,12 @@ inline hipError_t launch_fused(int prec, hipStream_t stream, const Scenario *sce
     if (prec == SW2D_FP64) return launch_fused_f64(stream, scen, tiles, nblocks, phase, features, lds);
     if (prec == SW2D_FP32) return launch_fused_f32(stream, scen, tiles, nblocks, phase, features, lds);
     return launch_fused_mix(stream, scen, tiles, nblocks, phase, features, lds);
+}
+inline hipError_t launch_forcing(int prec, hipStream_t stream, const Scenario *scen, int n)
+{
+    if (prec == SW2D_FP64) return launch_forcing_f64(stream, scen, n);
+    if (prec == SW2D_FP32) return launch_forcing_f32(stream, scen, n);
+    return launch_forcing_mix(stream, scen, n);
 }
 inline int fused_waves_per_cu(int prec, int features)
 {
