@@ -601,6 +601,10 @@ int sw2d_set_sources(sw2d_handle *h, const double *x, const double *y, int nst, 
         rr[i] = (int)(idx / h->C);
         cc[i] = (int)(idx % h->C);
     }
+    // no sources until all their arrays are there: after a failure no descriptor
+    // may name a released array (the clock wave of every iteration writes src_rate)
+    h->nst = h->nq = 0;
+    changed(h);
     int rc = upload_source_cells(h, rr.data(), cc.data(), nst);
     if (rc) return rc;
     dfree(h, h->Q);
