@@ -138,8 +138,10 @@ int sw2d_set_rain_series(sw2d_handle *h, const double *rain_mm, int n, double dt
  * (Q_source_sink.dat, 4041-4069).  The cell index uses stream_flow's formula
  * (541-544); values are evaluated on the device every half step (531-540),
  * replacing the dense ql upload of 4821 and 4845.  A source outside the
- * rows*cols real cells is an error.  The arrays of an earlier call are given
- * back first: after SW2D_E_NOMEM the handle has no sources. */
+ * rows*cols real cells is an error.
+ * This call and those for the rain and evaporation series, the hydrograph and
+ * the lake records give the arrays of an earlier call back first: after
+ * SW2D_E_NOMEM the handle has no sources (series, samples, records). */
 int sw2d_set_sources(sw2d_handle *h, const double *x, const double *y, int nst,
                      const double *Q, int nq, double dtoq);
 

@@ -565,6 +565,9 @@ int sw2d_set_rain_series(sw2d_handle *h, const double *rain_mm, int n, double dt
     if (n < 0 || (n > 0 && !rain_mm)) return fail(h, SW2D_E_ARG, "bad rain series");
     if (!(dtrain > 0)) return fail(h, SW2D_E_ARG, "dtrain must be positive");
     HIPCHK(h, hipStreamSynchronize(h->stream));
+    // no series until its array is there (as in sw2d_set_sources)
+    h->nrain = 0;
+    changed(h);
     dfree(h, h->rain);
     h->rain = nullptr;
     int rc = dalloc(h, &h->rain, n);
@@ -622,6 +625,8 @@ int sw2d_set_evaporation(sw2d_handle *h, const double *evapo_mm, int n)
     if (check_idle(h)) return SW2D_E_ARG;
     if (n < 0 || (n > 0 && !evapo_mm)) return fail(h, SW2D_E_ARG, "bad evaporation series");
     HIPCHK(h, hipStreamSynchronize(h->stream));
+    h->nevapo = h->evap_on = 0;
+    changed(h);
     dfree(h, h->evapo);
     h->evapo = nullptr;
     int rc = dalloc(h, &h->evapo, n);
@@ -692,6 +697,8 @@ int sw2d_set_hydrograph(sw2d_handle *h, long cap)
     if (check_idle(h)) return SW2D_E_ARG;
     if (cap < 0) return fail(h, SW2D_E_ARG, "negative capacity");
     HIPCHK(h, hipStreamSynchronize(h->stream));
+    h->hydro_cap = 0;
+    changed(h);
     dfree(h, h->hydro);
     h->hydro = nullptr;
     int rc = dalloc(h, &h->hydro, 2 * (size_t)cap);
@@ -721,6 +728,8 @@ int sw2d_set_lake_bc(sw2d_handle *h, const int *mask)
             br.push_back(p / C); bc.push_back(p % C); bk.push_back(k);
         }
     HIPCHK(h, hipStreamSynchronize(h->stream));
+    h->nbc = 0;
+    changed(h);
     dfree(h, h->bc_r); dfree(h, h->bc_c); dfree(h, h->bc_kind); dfree(h, h->bc_acc);
     h->bc_r = h->bc_c = h->bc_kind = nullptr;
     h->bc_acc = nullptr;

@@ -56,3 +56,64 @@ def test_sources(pkg, n, nq):
     for c in (member, alone):
         c.set_sources(*sources(5, 3))
     step_both(batch, member, alone, 8)
+
+
+def test_rain_and_evaporation(pkg):
+    batch, member, alone = pair(pkg)
+    for c in (member, alone):
+        c.set_rain(np.array([400.0, 100.0, 300.0]), 4.3)
+        c.set_evaporation(np.array([5.0, 9.0, 2.0]))
+    step_both(batch, member, alone, 3)
+    for setter, args in (("set_rain", (4.3,)), ("set_evaporation", ())):
+        with pytest.raises(pkg.sw2d.Sw2dError, match="pool exhausted"):
+            getattr(member, setter)(np.ones(300000), *args)
+        # a series without values gives the rate 0 between the interval ends
+        # (at one, where no step of 0.5 s comes, its formula divides 0 by 0)
+        getattr(alone, setter)(np.zeros(0), *args)
+        step_both(batch, member, alone, 8)
+    for c in (member, alone):
+        c.set_rain(np.array([200.0, 100.0, 50.0]), 9.0)
+    step_both(batch, member, alone, 8)
+
+
+def test_hydrograph(pkg):
+    batch, member, alone = pair(pkg)
+    for c in (member, alone):
+        c.set_outlet(SHAPE[0] - 1, 30)
+        c.set_hydrograph(40)
+    step_both(batch, member, alone, 3)
+    assert np.array_equal(member.hydrograph(), alone.hydrograph())
+    with pytest.raises(pkg.sw2d.Sw2dError, match="pool exhausted"):
+        member.set_hydrograph(100000)
+    alone.set_hydrograph(0)
+    step_both(batch, member, alone, 8)
+    assert len(member.hydrograph()) == 0
+    for c in (member, alone):
+        c.set_hydrograph(40)
+    step_both(batch, member, alone, 8)
+    assert np.array_equal(member.hydrograph()[11:], alone.hydrograph()[11:])
+
+
+# how many of the four arrays (4 bytes a record three times, then 8) find room
+@pytest.mark.parametrize("rooms", [0, 2, 3])
+def test_lake_records(pkg, rooms):
+    batch, member, alone = pair(pkg)
+    lake = np.zeros(SHAPE, np.int32)
+    lake[8:12, 20:40] = 1
+    for c in (member, alone):
+        c.set_lake_bc(lake)
+    step_both(batch, member, alone, 3)
+    assert np.array_equal(member.lake_inflow(), alone.lake_inflow())
+    many = (np.indices(SHAPE).sum(0) % 2).astype(np.int32)
+    alone.set_lake_bc(many)
+    assert alone.nbc > 1000
+    # another member's hydrograph takes the rest of the pool
+    z, h0 = terrain()
+    filler = batch.case(z, h0, DX, **KW)
+    used, _, cap = batch.memory()
+    left = rooms * (-(-4 * alone.nbc // 256) * 256) + 512
+    filler.set_hydrograph((cap - used - left) // 256 * 16)
+    with pytest.raises(pkg.sw2d.Sw2dError, match="pool exhausted"):
+        member.set_lake_bc(many)
+    step_both(batch, member, alone, 8)
+    assert len(member.lake_inflow()) == 0
