@@ -612,7 +612,8 @@ int sw2d_set_sources(sw2d_handle *h, const double *x, const double *y, int nst, 
     if (rc) return rc;
     dfree(h, h->Q);
     h->Q = nullptr;
-    if ((rc = dalloc(h, &h->Q, (size_t)nq * nst))) return rc;
+    // at least one row (of zeros): the rates at t <= 1 read it whatever nq is
+    if ((rc = dalloc(h, &h->Q, (size_t)std::max(nq, 1) * nst))) return rc;
     if ((size_t)nq * nst > 0)
         HIPCHK(h, hipMemcpy(h->Q, Q, sizeof(double) * nq * nst, hipMemcpyHostToDevice));
     h->nst = nst; h->nq = nq; h->dtoq = dtoq;

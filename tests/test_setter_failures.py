@@ -117,3 +117,15 @@ def test_lake_records(pkg, rooms):
         member.set_lake_bc(many)
     step_both(batch, member, alone, 8)
     assert len(member.lake_inflow()) == 0
+
+
+def test_sources_without_a_series_give_nothing(pkg):
+    """No rows in the table: the rates are 0 from the first step on, whatever
+    lies behind it in the pool (here the rain series).  No step comes at the
+    end of an interval, where the formula divides 0 by 0."""
+    batch, member, alone = pair(pkg)
+    x, y, _, _ = sources(100, 1)
+    member.set_sources(x, y, np.zeros((0, 100)), 7.3)
+    for c in (member, alone):
+        c.set_rain(np.full(400, 30.0), 7.3)
+    step_both(batch, member, alone, 8)
