@@ -61,27 +61,6 @@ size_t lds_for_cap(int device, int cap)
     return std::min<size_t>(per, prop.sharedMemPerBlock);
 }
 
-// the launch's tile table: each member's blocks in a run (order 0), or the
-// members interleaved block by block (order 1), so that every stretch of
-// the launch holds tiles of many members.  Either way the members' ledger
-// waves (block 0 of each), which are chains of loads, start first.
-void order_tiles(const std::vector<int> &counts, const std::vector<int> &sids, int order,
-                 std::vector<TileRef> &tiles)
-{
-    tiles.clear();
-    if (order == 0) {
-        for (size_t m = 0; m < counts.size(); m++) tiles.push_back(TileRef{sids[m], 0});
-        for (size_t m = 0; m < counts.size(); m++)
-            for (int i = 1; i < counts[m]; i++) tiles.push_back(TileRef{sids[m], i});
-        return;
-    }
-    int most = 0;
-    for (int c : counts) most = std::max(most, c);
-    for (int i = 0; i < most; i++)
-        for (size_t m = 0; m < counts.size(); m++)
-            if (i < counts[m]) tiles.push_back(TileRef{sids[m], i});
-}
-
 // descriptors and tile table of the attached members
 int rebuild(sw2d_batch *b)
 {

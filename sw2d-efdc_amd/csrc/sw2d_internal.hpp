@@ -23,6 +23,7 @@
 
 #include "../../include/sw2d.h"
 #include "sw2d_pool.hpp"
+#include "sw2d_schedule.hpp"
 
 namespace sw2d {
 
@@ -158,21 +159,11 @@ struct Scenario {
     Status *status;          // batch members only; NULL for a stand-alone handle
 };
 
-// bookkeeping waves besides those of the lake-inflow records (64 each): the
-// clock and the forcing, the ledger
-constexpr int kBookParts = 2;
-inline int book_blocks(int nbc) { return kBookParts + (nbc + 63) / 64; }
-
 // tile height of batch members that name none: between what
 // ensembles that fill the chip for several rounds and smaller ones want (a launch
 // of 24 grids of 128^2..1024^2 in FP64 takes 133 us at 20 rows, 147 at 32, 137 at
 // 12; 48 of them in FP32 108, 112, 113)
 constexpr int kBatchTileRows = 20;
-
-// one block of a batched launch: scenario and block within it
-struct TileRef {
-    int sid, local;
-};
 
 // Features of a scenario that the fused kernel can compile out where no
 // scenario of a launch uses them.
