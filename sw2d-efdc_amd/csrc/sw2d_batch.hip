@@ -49,16 +49,16 @@ hipError_t blaunch(sw2d_batch *b, const Scenario *scen, const TileRef *tiles, in
     return launch_fused(b->precision, b->stream, scen, tiles, nblocks, phase, features, b->lds_pad);
 }
 
-// unused LDS per one-wave block that leaves room for at most `cap` resident
-// blocks per SIMD (four SIMDs per CU); 0 for no cap
-size_t lds_for_cap(int device, int cap)
+// unused LDS per one-wave block of the kernel that runs `features`, which leaves
+// room for at most `cap` resident blocks per SIMD; 0 for no cap
+size_t lds_for_cap(int device, int prec, int features, int cap)
 {
     if (cap <= 0) return 0;
-    hipDeviceProp_t prop;
-    if (hipGetDeviceProperties(&prop, device) != hipSuccess) return 0;
-    size_t per = prop.maxSharedMemoryPerMultiProcessor / (4 * (size_t)cap);
-    per = per / 256 * 256;
-    return std::min<size_t>(per, prop.sharedMemPerBlock);
+    int per_cu = 0, per_block = 0;
+    if (hipDeviceGetAttribute(&per_cu, hipDeviceAttributeMaxSharedMemoryPerMultiprocessor, device) != hipSuccess ||
+        hipDeviceGetAttribute(&per_block, hipDeviceAttributeMaxSharedMemoryPerBlock, device) != hipSuccess)
+        return 0;
+    return lds_pad((size_t)per_cu, (size_t)per_block, fused_lds(prec, features), cap);
 }
 
 // descriptors and tile table of the attached members
@@ -102,9 +102,11 @@ int rebuild(sw2d_batch *b)
     }
     if (!tiles.empty())
         BCHK(b, hipMemcpy(b->dtiles, tiles.data(), sizeof(TileRef) * tiles.size(), hipMemcpyHostToDevice));
-    if ((int)tiles.size() != b->nblocks || features != b->features) bdrop_graph(b);
+    const size_t pad = lds_for_cap(b->device, b->precision, features, b->waves_cap);
+    if ((int)tiles.size() != b->nblocks || features != b->features || pad != b->lds_pad) bdrop_graph(b);
     b->nblocks = (int)tiles.size();
     b->features = features;
+    b->lds_pad = pad;
     b->dirty = false;
     return SW2D_OK;
 }
@@ -506,7 +508,7 @@ int sw2d_batch_autotune(sw2d_batch *b, int iters, int *tile_rows)
         order_tiles(counts, sids, order, tiles);
         if (e != hipSuccess || tiles.empty()) return -1.0f;
         const size_t lds_live = b->lds_pad;
-        b->lds_pad = lds_for_cap(b->device, cap);
+        b->lds_pad = lds_for_cap(b->device, b->precision, feats, cap);
         e = hipMemcpy(dscen_s, desc.data(), sizeof(Scenario) * nm, hipMemcpyHostToDevice);
         if (e == hipSuccess) e = hipMemcpy(dtiles_s, tiles.data(), sizeof(TileRef) * tiles.size(), hipMemcpyHostToDevice);
         if (e == hipSuccess) e = blaunch(b, dscen_s, dtiles_s, (int)tiles.size(), phase, feats);
@@ -569,7 +571,6 @@ int sw2d_batch_autotune(sw2d_batch *b, int iters, int *tile_rows)
     if (best_order != b->order || best_cap != b->waves_cap) {
         b->order = best_order;
         b->waves_cap = best_cap;
-        b->lds_pad = lds_for_cap(b->device, best_cap);
         bdrop_graph(b);
     }
     // retiling folds each member's pending partial sums into one record
@@ -591,7 +592,6 @@ int sw2d_batch_set_schedule(sw2d_batch *b, int order, int waves_per_simd)
     BCHK(b, hipStreamSynchronize(b->stream));
     b->order = order;
     b->waves_cap = waves_per_simd;
-    b->lds_pad = lds_for_cap(b->device, waves_per_simd);
     bdrop_graph(b);
     b->dirty = true;
     return SW2D_OK;

@@ -44,6 +44,7 @@ hipError_t launch_forcing_f32(hipStream_t stream, const Scenario *scen, int n)
     return launch_forcing_impl<float, float>(stream, scen, n);
 }
 int fused_waves_per_cu_f32(int features) { return fused_waves_per_cu_impl<float, float>(features); }
+size_t fused_lds_f32(int features) { return fused_lds_impl<float, float>(features); }
 hipError_t launch_init_f32(sw2d_handle *h) { return launch_init_impl<float, float>(h); }
 hipError_t launch_bed_steps(sw2d_handle *h)
 {

@@ -20,6 +20,7 @@ hipError_t launch_forcing_f64(hipStream_t stream, const Scenario *scen, int n)
     return launch_forcing_impl<double, double>(stream, scen, n);
 }
 int fused_waves_per_cu_f64(int features) { return fused_waves_per_cu_impl<double, double>(features); }
+size_t fused_lds_f64(int features) { return fused_lds_impl<double, double>(features); }
 hipError_t launch_init_f64(sw2d_handle *h) { return launch_init_impl<double, double>(h); }
 hipError_t launch_derive_f64(sw2d_handle *h, int field, double *out, long first, long count)
 {

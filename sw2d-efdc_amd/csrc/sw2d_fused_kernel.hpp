@@ -945,21 +945,35 @@ static hipError_t launch_fused_impl(hipStream_t stream, const Scenario *scen, co
     return hipGetLastError();
 }
 
-// resident one-wave blocks per CU of the instantiation that runs `features`
+// the instantiation that runs `features`
+template <typename T, typename TH>
+static const void *fused_fn(int features)
+{
+    switch (fused_variant(features)) {
+    case kVariant0: return (const void *)fused_step<T, TH, kVariant0>;
+    case kVariant1: return (const void *)fused_step<T, TH, kVariant1>;
+    case kVariant2: return (const void *)fused_step<T, TH, kVariant2>;
+    case kVariant3: return (const void *)fused_step<T, TH, kVariant3>;
+    default: return (const void *)fused_step<T, TH, kFeatAll>;
+    }
+}
+
+// its resident one-wave blocks per CU
 template <typename T, typename TH>
 static int fused_waves_per_cu_impl(int features)
 {
-    const void *fn;
-    switch (fused_variant(features)) {
-    case kVariant0: fn = (const void *)fused_step<T, TH, kVariant0>; break;
-    case kVariant1: fn = (const void *)fused_step<T, TH, kVariant1>; break;
-    case kVariant2: fn = (const void *)fused_step<T, TH, kVariant2>; break;
-    case kVariant3: fn = (const void *)fused_step<T, TH, kVariant3>; break;
-    default: fn = (const void *)fused_step<T, TH, kFeatAll>; break;
-    }
     int nb = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, fn, 64, 0) != hipSuccess) return 0;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, fused_fn<T, TH>(features), 64, 0) != hipSuccess) return 0;
     return nb;
+}
+
+// its blocks' own LDS (the tables, the clipped volume, the storm's rows)
+template <typename T, typename TH>
+static size_t fused_lds_impl(int features)
+{
+    hipFuncAttributes a;
+    if (hipFuncGetAttributes(&a, fused_fn<T, TH>(features)) != hipSuccess) return 0;
+    return a.sharedSizeBytes;
 }
 
 template <typename T, typename TH>

@@ -19,6 +19,7 @@ hipError_t launch_forcing_mix(hipStream_t stream, const Scenario *scen, int n)
     return launch_forcing_impl<float, double>(stream, scen, n);
 }
 int fused_waves_per_cu_mix(int features) { return fused_waves_per_cu_impl<float, double>(features); }
+size_t fused_lds_mix(int features) { return fused_lds_impl<float, double>(features); }
 hipError_t launch_init_mix(sw2d_handle *h) { return launch_init_impl<float, double>(h); }
 hipError_t launch_derive_mix(sw2d_handle *h, int field, double *out, long first, long count)
 {

@@ -285,7 +285,7 @@ struct sw2d_batch {
     // launch schedule (sw2d_batch_set_schedule): block order 0 = each
     // member's tiles in a run, 1 = members interleaved tile by tile; a cap
     // on resident waves per SIMD (0 = none), enforced by reserving lds_pad
-    // bytes of unused LDS per one-wave block
+    // bytes of unused LDS per one-wave block (set by rebuild)
     int order = 0;
     int waves_cap = 0;
     size_t lds_pad = 0;
@@ -344,6 +344,9 @@ hipError_t launch_forcing_mix(hipStream_t stream, const Scenario *scen, int n);
 int fused_waves_per_cu_f64(int features);  // resident one-wave blocks per CU
 int fused_waves_per_cu_f32(int features);
 int fused_waves_per_cu_mix(int features);
+size_t fused_lds_f64(int features);        // LDS of a block of its own
+size_t fused_lds_f32(int features);
+size_t fused_lds_mix(int features);
 
 // bytes of a stored depth and of a stored face flux in a precision form
 inline int depth_bytes(int prec) { return prec == SW2D_FP32 ? 4 : 8; }
@@ -372,6 +375,12 @@ inline int fused_waves_per_cu(int prec, int features)
     if (prec == SW2D_FP64) return fused_waves_per_cu_f64(features);
     if (prec == SW2D_FP32) return fused_waves_per_cu_f32(features);
     return fused_waves_per_cu_mix(features);
+}
+inline size_t fused_lds(int prec, int features)
+{
+    if (prec == SW2D_FP64) return fused_lds_f64(features);
+    if (prec == SW2D_FP32) return fused_lds_f32(features);
+    return fused_lds_mix(features);
 }
 hipError_t launch_plain(sw2d_handle *h, const StepCommon &sc);
 hipError_t launch_plain_init(sw2d_handle *h);
