@@ -325,8 +325,10 @@ fused_step(const Scenario *__restrict__ scen, const TileRef *__restrict__ tiles,
         pow_s[64 + lane] = kPowNlog[lane];
         pow_s[128 + lane] = kPowExp2[lane];
         if (lane < 16) pow_s[192 + lane] = kPowCoefMem[lane];
-        __syncthreads();
     }
+    // lanes read what others wrote (the block is one wave: this orders, it does
+    // not wait)
+    if constexpr (kMap || !kF32) __syncthreads();
     const int kbeg = r0 - 3, kend = r1 + 3, kload = kend < R ? kend : R;
     // Row to load next: its offset (in elements), and the lanes' byte offsets.
     // While that row is outside the grid (or past the last one that is needed)
