@@ -198,7 +198,7 @@ constexpr int kMaxTileRows = 512;
 // 3 against 2 in FP64: 2048^2 134 -> 125 us when it came; 4 (128 registers) spill:
 // 107 -> 137.  5 against 4 in FP32: 2048^2 59.0 -> 56.8 when it came; 6 (80
 // registers) spill in the storm's instantiation: 50.4 -> 53.1.
-template <typename T, int F>
+template <typename T>
 constexpr int kMinWaves = (sizeof(T) == 8 ? 3 : 5);
 
 // F: the features (kFeat*) this instantiation handles.  A feature missing
@@ -208,7 +208,7 @@ constexpr int kMinWaves = (sizeof(T) == 8 ? 3 : 5);
 // multiply-add, FP32 only within one source expression), so a scenario's
 // results do not depend on the instantiation that ran it.
 template <typename T, typename TH, int F>
-__global__ void __launch_bounds__(64, (kMinWaves<T, F>))
+__global__ void __launch_bounds__(64, (kMinWaves<T>))
 fused_step(const Scenario *__restrict__ scen, const TileRef *__restrict__ tiles, const int nblocks,
            const int phase)
 {

@@ -37,10 +37,6 @@ inline bool graphs_enabled()
     return !(e && e[0] == '0');
 }
 
-// pointer into global memory (address space 1 of the AMDGPU target)
-template <typename T>
-using gptr = __attribute__((address_space(1))) T *;
-
 constexpr unsigned long long kInfBits = 0x7ff0000000000000ULL;
 constexpr int kMaxClasses = 8;
 

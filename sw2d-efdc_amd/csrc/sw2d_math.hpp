@@ -252,8 +252,6 @@ template <> struct num<double> {
     __device__ static __forceinline__ double max_(double a, double b) { return __builtin_fmax(a, b); }
     __device__ static __forceinline__ double exp_(double x) { return exp_d(x); }
     __device__ static __forceinline__ double div_(double a, double b) { return a / b; }
-    // x / |x| for nonzero finite x (exactly +-1)
-    __device__ static __forceinline__ double sign_(double x) { return __builtin_copysign(1.0, x); }
     // a / b where rb = 1 / b is precomputed (FP64 still divides)
     __device__ static __forceinline__ double divc_(double a, double b, double rb) { return a / b; }
 };
@@ -263,7 +261,6 @@ template <> struct num<float> {
     __device__ static __forceinline__ float max_(float a, float b) { return __builtin_fmaxf(a, b); }
     __device__ static __forceinline__ float exp_(float x) { return exp_f(x); }
     __device__ static __forceinline__ float div_(float a, float b) { return a * __builtin_amdgcn_rcpf(b); }
-    __device__ static __forceinline__ float sign_(float x) { return __builtin_copysignf(1.0f, x); }
     __device__ static __forceinline__ float divc_(float a, float b, float rb) { return a * rb; }
 };
 
