@@ -331,7 +331,8 @@ typedef struct sw2d_batch sw2d_batch;
 
 /* A batch on `device` owns one stream and a device memory pool of
  * pool_bytes; every member's arrays come from the pool.  All members share
- * `precision`.  tile_rows: rows per tile of members (0 = automatic). */
+ * `precision`.  tile_rows: rows per tile that members start at (0 = 20;
+ * sw2d_batch_autotune measures the height for the members at hand). */
 int sw2d_batch_create(int device, int precision, size_t pool_bytes, int tile_rows, sw2d_batch **out);
 /* Destroys the members still in the batch, then the batch. */
 int sw2d_batch_destroy(sw2d_batch *b);
@@ -459,8 +460,8 @@ typedef struct sw2d_server_stats {
  * after each admission or retirement the running requests are retiled to the
  * height that fills whole rounds of wave slots, the fewest rounds with a
  * height of at most 80, else 32, or where their launch is bound by memory to
- * the one a model of the kernel finds shortest; results are those of any fixed height, the
- * volume ledger to rounding).
+ * the one a model of the kernel finds shortest; results are those of any
+ * fixed height, the volume ledger to rounding).
  * slice_iters: iterations per batch step between admissions (0 = 60).
  * The server's batch interleaves the running requests' tiles block by block
  * (sw2d_batch_set_schedule order 1).

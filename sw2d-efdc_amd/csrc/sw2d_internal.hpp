@@ -158,7 +158,9 @@ struct Scenario {
 // tile height of batch members that name none: between what
 // ensembles that fill the chip for several rounds and smaller ones want (a launch
 // of 24 grids of 128^2..1024^2 in FP64 takes 133 us at 20 rows, 147 at 32, 137 at
-// 12; 48 of them in FP32 108, 112, 113)
+// 12; 48 of them in FP32 108, 112, 113; 6 of them 52 and 31 us at 20 rows in FP64
+// and FP32, 52 and 28 at 8, 71 and 43 at 32; 256 of them 1107 and 496 at 20, 1064
+// and 541 at 32)
 constexpr int kBatchTileRows = 20;
 
 // Features of a scenario that the fused kernel can compile out where no

@@ -21,7 +21,9 @@ inline int book_blocks(int nbc) { return kBookParts + (nbc + 63) / 64; }
 // the launch's tile table: each member's blocks in a run (order 0), or the
 // members interleaved block by block (order 1), so that every stretch of
 // the launch holds tiles of many members.  Either way the members' clock and
-// ledger waves, which are chains of loads, start first.
+// ledger waves, which are chains of loads, start first (24 grids of 128^2..1024^2
+// in FP64 134.5 us a launch with the clock waves alone there, 134.1 with both; 48
+// in FP32 108.4 and 108.2).
 inline void order_tiles(const std::vector<int> &counts, const std::vector<int> &sids, int order,
                         std::vector<TileRef> &tiles)
 {

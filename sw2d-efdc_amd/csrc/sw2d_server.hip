@@ -9,9 +9,10 @@
 // request that arrives while others run starts at the next slice boundary
 // instead of waiting for the GPU to drain.  With adaptive tiling the running
 // set is retiled after each change of membership to the height that fills
-// whole rounds of wave slots: a few small requests run as many short tiles
-// (their time per iteration is the tile's row chain), a full GPU as fewer,
-// taller ones (fewer halo rows re-read).
+// whole rounds of wave slots, or, where memory bounds the launch, to the one
+// that the model of the row loop finds shortest: a few small requests run as
+// many short tiles (their time per iteration is the tile's row chain), a full
+// GPU as fewer, taller ones (fewer halo rows re-read).
 #include <math.h>
 #include <stdlib.h>
 

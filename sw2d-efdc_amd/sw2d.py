@@ -588,7 +588,9 @@ class Batch:
 class Server:
     """Continuous-batching request loop on a device thread (sw2d_server_*).
     tile_rows=0 retiles the running requests after each admission or
-    retirement to the height that fills whole rounds of wave slots."""
+    retirement to the height that fills whole rounds of wave slots, or, where
+    memory bounds the launch, to the one that a model of the kernel finds
+    shortest."""
 
     def __init__(self, precision="fp32", pool_bytes=8 << 30, tile_rows=0, slice_iters=60,
                  max_active_cells=0, device=0):
